@@ -4,13 +4,13 @@
 // cda/kernels_cuda/wrappers.py:79-124; math of cda/algorithm/attention.py:
 // 426-482 (attention_compressed), split-K partials and merge of :190-272.
 //
-// Default form, one launch (decode_stream_kernel<..., FUSED = true>): where
-// the page-streaming kernel applies (8 KV heads, 144- or 80-byte slots, one
-// codebook pointer, the library's split plan), one workgroup per (sequence,
-// context split, KV head) rotates that head's GQA group of q, streams the
-// head's pages on eight waves over consecutive token ranges, merges the
-// waves' partials in LDS and, when one split covers the sequence, applies
-// R^T and writes out; with several splits the combine launch follows.
+// Default form, one launch (decode_stream_kernel<..., FUSED = true>): K4V4 and
+// K2V2 caches of any head count and slot width (a multiple of 16), with the
+// library's split plan.  One workgroup per (sequence, context split, KV head)
+// rotates that head's GQA group of q, streams the head's pages on eight waves
+// over consecutive token ranges, merges the waves' partials in LDS and, when
+// one split covers the sequence, applies R^T and writes out; with several
+// splits the combine launch follows.
 //
 // Otherwise three launches on the caller's stream:
 //   1. rotate_q:  q_rot = fp16(q @ R) per (b, q-head).
@@ -92,7 +92,7 @@ struct SplitParams {
     const float *R;             // (128, 128) fp32 rotation
     uint16_t *out;              // (B, H_q, 128) fp16
     int wave_tokens;            // multiple of 64
-    int xcd_map;                // 1: the 8 heads of a (sequence, split) share an XCD
+    int xcd_map;                // 1: the heads of a (sequence, split) share an XCD
 };
 
 __device__ __forceinline__ floatx4 mfma16(uint4 a, uint4 b, floatx4 c) {
@@ -476,34 +476,36 @@ decode_split_kernel(SplitParams p) {
 }
 
 // ---------------------------------------------------------------------------
-// Page-streaming split kernel for the common cache shapes: 8 KV heads x
-// 144-byte K4V4 slots (L = 16) or 80-byte K2V2 slots (L = 4), a block size
-// that is a multiple of 16 and one codebook for K and V.  The K4V4 layout is
-// described first; the K2V2 differences follow.
+// Page-streaming kernel for K4V4 (L = 16) and K2V2 (L = 4) slots and a block
+// size that is a multiple of 16.  Its three-launch form needs 8 KV heads (one
+// per wave), 144- or 80-byte slots and one codebook for K and V; the
+// single-launch form (FUSED, below) does not.  The K4V4 layout is described
+// first; the K2V2 differences follow.
 //
 // Wave h (one per KV head) streams its head's share of each 16-token page
 // (16 x 144 B = 2304 B) into a private 4-page LDS ring with the gfx950
-// direct-to-LDS DMA (buffer_load_dwordx4 ... lds): three instructions per page
-// (K codes, V codes, norms), each lane fetching one 16-byte piece.  The waves
+// direct-to-LDS DMA (buffer_load_dwordx4 ... lds): three instructions per page,
+// each lane fetching one 16-byte piece.  Consecutive lanes take consecutive
+// pieces of a token's slot (piece p = token p / 9, bytes 16 * (p % 9)), so a
+// slot is fetched as the two cache lines it lies on; one instruction each for
+// the K codes, V codes and norms touches 3.75 lines per token.  The waves
 // never wait for each other: each one waits on its own DMA counter only.  A
 // step takes a chunk of four pages (64 tokens): wait for the chunk's DMAs,
 // read the four pages into registers, refill the four slots with the next
 // chunk (in flight while this one computes), then QK^T on the four pages
 // (independent MFMA chains), one online-softmax update over the 64 tokens and
 // PV over two page pairs.  Page k of a chunk lives in ring slot k, so every
-// ring offset is an immediate.  Within a page the pieces are laid out so that
-// every read is free of LDS bank conflicts:
-//   [0, 1024)     K codes: piece 16*c + t = token t, 16-byte column c (0..3)
-//   [1024, 2048)  V codes: token t's 64 bytes at 64 * vslot(t)
-//   [2048, 2304)  norms:   token t's (Kn, Vn, pad) at 16 * t
+// ring offset is an immediate.  A ring page is the 16 slots in token order,
+// 144 bytes apart, and every read of it is free of LDS bank conflicts (64
+// banks of 4 bytes): 144 * t mod 256 takes 16 different multiples of 16 for the
+// 16 tokens of a K read, and tokens 4 * q4 + i (q4 = 0..3) of a V read start 64
+// bytes apart.
 // One dequant table serves K and V: row e (256 B) holds (cb[e >> 4],
 // cb[e & 15]) in fp32 for 32 lane columns, read with one ds_read_b64 per code
 // byte.
 //
-// K2V2 (1280 B per head and page, two DMA instructions):
-//   [0, 512)      K codes: piece 16*c + t = token t, 16-byte column c (0..1)
-//   [512, 1024)   V codes: token t's 32 bytes at 32 * vslot2(t)
-//   [1024, 1280)  norms, as above
+// K2V2: 1280 B per head and page, five pieces per token, two DMA instructions;
+// slots 80 bytes apart, with the same bank property.
 // The table row e (256 B) holds, for 16 lane columns of 16 bytes,
 // (cb[e >> 6], cb[(e >> 4) & 3], cb[(e >> 2) & 3], cb[e & 3]): a byte of
 // 2-bit codes (dims 4j..4j+3, first dim in bits 7:6) gives its four values in
@@ -543,11 +545,6 @@ __device__ __forceinline__ uint32_t lds_b32(const uint8_t *base, uint32_t off) {
     return *reinterpret_cast<const uint32_t *>(base + off);
 }
 
-// 64-byte V slot of token t within its group of four: the four tokens read
-// together (4*q4 + i, q4 = 0..3) land in four different bank quarters.
-__host__ __device__ constexpr int vslot(int t) { return (t & 12) | ((t + (t >> 2)) & 3); }
-__host__ __device__ constexpr int vslot_inv(int s) { return (s & 12) | ((s - (s >> 2)) & 3); }
-
 // The score-domain form (SQK) bounds the drift between its waves with a
 // workgroup barrier every 8 chunks: with the lighter K side it is bound by the
 // fetched bytes, and waves that drift apart fetch the 64-byte segments shared
@@ -567,10 +564,6 @@ constexpr int kFusedQrOff = kFusedQOff + 8 * kD * 4;
 constexpr int kFusedLds = kFusedQrOff + 8 * kD * 2;                         // 159744 B
 static_assert(kFusedLds <= 160 * 1024, "FUSED LDS");
 
-// K2V2 V slot of token t: the four tokens read together (4*q4 + i, q4 =
-// 0..3) land in four consecutive 32-byte slots (an involution).
-__host__ __device__ constexpr int vslot2(int t) { return ((t & 3) << 2) | (t >> 2); }
-
 // Bit-field insert: bits of a where m is set, of b elsewhere (v_bfi_b32).
 __device__ __forceinline__ uint32_t bfi(uint32_t m, uint32_t a, uint32_t b) {
     return (m & a) | (~m & b);
@@ -582,13 +575,25 @@ __device__ __forceinline__ uint32_t bfi(uint32_t m, uint32_t a, uint32_t b) {
 // code (the subnormal code * 2^-24, exact; no table, no multiply), so
 // q_rot . code = acc * 2^24 exactly up to fp32 accumulation; V is decoded
 // as in the default form, through a table of cb_v.
-template <int GS, int L, bool SQK = false, bool FUSED = false>
+//
+// FUSED: the single-launch form.  A workgroup owns one KV head, so it takes any
+// head count and any slot of at least S bytes (a multiple of 16): only the row
+// and slot strides change, the bytes copied into LDS are the same.
+//
+// TWO (FUSED only): K and V have a codebook each.  Both tables share the 64 KiB:
+// a 256-byte row holds the K entry in the first half of the lane columns and
+// the V entry in the second, so a table read is the same instruction with an
+// offset of 128.  With half the columns two lanes of a read share each bank:
+// 4.0 instead of 2.9 cycles per ds_read_b64 and CU, 8.2 instead of 4.1 per
+// ds_read_b128 (2-bit codes), which is why one codebook keeps the full row.
+template <int GS, int L, bool SQK = false, bool FUSED = false, bool TWO = false>
 __global__ void __launch_bounds__(kThreads, 1)
 decode_stream_kernel(SplitParams p) {
     if (!FUSED && !SQK && p.cb_same && !*p.cb_same) return;   // different codebooks: the general kernel runs
     static_assert(L == 16 || L == 4, "4-bit or 2-bit codes");
     static_assert(!SQK || L == 16, "score-domain QK: 4-bit K codes");
     static_assert(!(SQK && FUSED), "the score-domain form runs as three launches");
+    static_assert(FUSED || !TWO, "two codebooks: single-launch form");
     static_assert(GS == 4 || GS == 8, "GQA groups of 4 or 8");
     // The MFMA's 16 score columns hold the GS heads RP times over, so every
     // lane holds every score of its head RP times.  Each lane computes the
@@ -597,13 +602,10 @@ decode_stream_kernel(SplitParams p) {
     constexpr int RP = 16 / GS;
     constexpr int NPL = 4 / RP;
     __shared__ __align__(16) uint8_t smem[FUSED ? kFusedLds : kStreamLds];
-    constexpr int S = (L == 16) ? 144 : 80;        // slot bytes
+    constexpr int S = (L == 16) ? 144 : 80;        // bytes of a slot copied into LDS
     constexpr int KB = (L == 16) ? 64 : 32;        // code bytes per role
-    constexpr int kRow = 8 * S;                    // one token row, all heads
-    constexpr int kPB = 16 * kRow;                 // one 16-token page, all heads
+    const int row_bytes = (int)p.row_bytes;        // one token row, all heads
     constexpr int kHP = 16 * S;                    // one head's share of a page
-    constexpr uint32_t kVo = 16 * KB;              // V codes within a ring page
-    constexpr uint32_t kNo = 32 * KB;              // norms within a ring page
     static_assert(kWaves * kStreamPages * kHP + kStreamRingOff <= kStreamPidOff, "ring fits");
 
     const int tid = threadIdx.x;
@@ -615,17 +617,17 @@ decode_stream_kernel(SplitParams p) {
     if constexpr (FUSED) {
         // Linear id -> (unit = (sequence, split), head).  The hardware deals
         // workgroups to the 8 XCDs round-robin by linear id; with xcd_map the
-        // 8 heads of a unit go to one XCD, so the 64-byte segments that
-        // neighbouring heads' slots share are fetched into one L2.
+        // heads of a unit go to one XCD, so the cache lines that neighbouring
+        // heads' slots share are fetched into one L2.
         const int pl = blockIdx.x;
         int u;
         if (p.xcd_map) {
             const int i = pl >> 3;
-            h = i & 7;
-            u = ((i >> 3) << 3) + (pl & 7);
+            h = i % p.H_kv;
+            u = (i / p.H_kv) * 8 + (pl & 7);
         } else {
-            h = pl & 7;
-            u = pl >> 3;
+            h = pl % p.H_kv;
+            u = pl / p.H_kv;
         }
         sp = u % p.n_splits;
         b = u / p.n_splits;
@@ -668,19 +670,16 @@ decode_stream_kernel(SplitParams p) {
         return;
     }
 
-    // Source offset of lane's 16-byte piece within the head's page rows.
-    uint32_t src[3];
-    if constexpr (L == 16) {
-        src[0] = (uint32_t)((lane & 15) * kRow + (lane >> 4) * 16);
-        src[1] = (uint32_t)(vslot_inv(lane >> 2) * kRow + KB + (lane & 3) * 16);
-        src[2] = (uint32_t)((lane & 15) * kRow + 2 * KB);   // lanes 0..15 only
-    } else {
-        // lanes 0..31: K pieces; lanes 32..63: V pieces (LDS 512 + 16*(lane-32)).
-        const int j = lane & 31;
-        src[0] = (lane < 32) ? (uint32_t)((j & 15) * kRow + (j >> 4) * 16)
-                             : (uint32_t)(vslot2(j >> 1) * kRow + KB + (j & 1) * 16);
-        src[2] = (uint32_t)((lane & 15) * kRow + 2 * KB);   // lanes 0..15 only
-        src[1] = 0;
+    // Source offset of this lane's piece of each DMA instruction within the
+    // head's page rows: piece 64 * i + lane of the page's 16 * kPieces.
+    constexpr int kPieces = S / 16;                // 16-byte pieces of a slot: 9 or 5
+    constexpr int kDma = (16 * kPieces + 63) / 64; // DMA instructions per page
+    static_assert(16 * kPieces % 64 == 16, "the last instruction moves 16 pieces");
+    uint32_t src[kDma];
+#pragma unroll
+    for (int i = 0; i < kDma; ++i) {
+        const int piece = 64 * i + lane;
+        src[i] = (uint32_t)((piece / kPieces) * row_bytes + (piece % kPieces) * 16);
     }
 
     const int bs = p.block_size;
@@ -697,17 +696,18 @@ decode_stream_kernel(SplitParams p) {
             page_row[t] = bt[t0 / bs] * bs + (t0 % bs);
         }
     }
-    const uint8_t *kv_h = p.kv + h * S;
+    const uint8_t *kv_h = p.kv + (int64_t)h * p.slot_bytes;
+    const uint32_t page_bytes = (uint32_t)(16 * row_bytes - h * p.slot_bytes);
     // DMA of the page starting at cache row row0 into ring slot k.
     auto issue_row = [&](int64_t row0, int k) CDA_INLINE {
-        const uint64_t base = (uint64_t)(kv_h + row0 * kRow);
+        const uint64_t base = (uint64_t)(kv_h + row0 * row_bytes);
         const v4u32 r = {(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)base),
                          (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(base >> 32) & 0xFFFFu),
-                         (uint32_t)(kPB - h * S), 0x00020000u};
+                         page_bytes, 0x00020000u};
         const uint32_t sb = ring_w + (uint32_t)k * kHP;
-        dma_page_chunk(r, src[0], sb);
-        if constexpr (L == 16) dma_page_chunk(r, src[1], sb + kVo);
-        if (lane < 16) dma_page_chunk(r, src[2], sb + kNo);
+#pragma unroll
+        for (int i = 0; i < kDma - 1; ++i) dma_page_chunk(r, src[i], sb + 1024u * i);
+        if (lane < 16) dma_page_chunk(r, src[kDma - 1], sb + 1024u * (kDma - 1));
     };
     // DMA of page t (row from the workgroup's table) into ring slot k.
     auto issue = [&](int t, int k) CDA_INLINE {
@@ -754,16 +754,18 @@ decode_stream_kernel(SplitParams p) {
         // The codebook goes through LDS first: a global load per table entry
         // would put 32 dependent memory round trips in every thread's
         // prologue.
-        __shared__ float cbs[16];
+        __shared__ float cbs[TWO ? 32 : 16];
         if (tid < L) cbs[tid] = SQK ? p.cb_v[tid] : p.cb_k[tid];
+        if (TWO && tid >= 16 && tid < 16 + L) cbs[tid] = p.cb_v[tid - 16];
         __syncthreads();
         uint32_t *lut = reinterpret_cast<uint32_t *>(smem);
         for (int i = tid; i < kLut2Bytes / 4; i += kThreads) {
             const int e = i >> 6;
+            const float *cb = cbs + (TWO ? (i & 32) >> 1 : 0);   // second half of a row: V
             if constexpr (L == 16)
-                lut[i] = __float_as_uint(cbs[(i & 1) ? (e & 15) : (e >> 4)]);
+                lut[i] = __float_as_uint(cb[(i & 1) ? (e & 15) : (e >> 4)]);
             else   // quad q of row e: the code in bits 7-2q:6-2q (dims 4j + q)
-                lut[i] = __float_as_uint(cbs[(e >> (6 - 2 * (i & 3))) & 3]);
+                lut[i] = __float_as_uint(cb[(e >> (6 - 2 * (i & 3))) & 3]);
         }
     }
     if constexpr (FUSED) {
@@ -790,21 +792,19 @@ decode_stream_kernel(SplitParams p) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
     const uint32_t rb0 = (uint32_t)(kStreamRingOff + wave * (kStreamPages * kHP));
-    // K4V4: token r16's 16 code bytes of dims [32*q4, +32); K2V2: its 8 bytes.
-    const uint32_t oK = (L == 16) ? rb0 + (uint32_t)lane * 16u
-                                  : rb0 + 256u * (q4 >> 1) + 16u * r16 + 8u * (q4 & 1);
-    const uint32_t oNK = rb0 + kNo + 16u * r16;
-    uint32_t oV[4], oNV[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        oV[i] = (L == 16) ? rb0 + kVo + 64u * vslot(4 * q4 + i) + 4u * r16
-                          : rb0 + kVo + 32u * vslot2(4 * q4 + i) + 2u * r16;
-        oNV[i] = rb0 + kNo + 16u * (4 * q4 + i) + 4u;
-    }
+    // Token r16's code bytes of dims [32*q4, +32) and its K norm; the V codes
+    // and V norm of tokens 4*q4 + i (i * S further on).
+    const uint32_t oK = rb0 + (uint32_t)(S * r16 + KB / 4 * q4);
+    const uint32_t oNK = rb0 + (uint32_t)(S * r16 + 2 * KB);
+    const uint32_t oV = rb0 + (uint32_t)(S * 4 * q4 + KB + KB / 16 * r16);
+    const uint32_t oNV = rb0 + (uint32_t)(S * 4 * q4 + 2 * KB + 4);
     // Table column of this lane: 32 columns of 8-byte pairs (4-bit codes) or
     // 16 columns of 16-byte quads (2-bit codes); either way a row is 256 bytes.
-    const uint32_t col = (L == 16) ? (uint32_t)(lane & 31) * 8u : (uint32_t)(lane & 15) * 16u;
+    // With two codebooks K takes the first half of the columns, V the second.
+    const uint32_t col = (L == 16) ? (uint32_t)(lane & (TWO ? 15 : 31)) * 8u
+                                   : (uint32_t)(lane & (TWO ? 7 : 15)) * 16u;
     const uint8_t *lutb = smem;
+    constexpr int kVTab = TWO ? 128 : 0;
     const int g_own = r16 / GS;
 
     floatx4 acc_o[8];
@@ -814,6 +814,8 @@ decode_stream_kernel(SplitParams p) {
     float l_run = 0.0f;
 
 #define CDA_PAIR(K_, W_) (*reinterpret_cast<const float2 *>(lutb + lut_addr<K_>(W_, col)))
+#define CDA_PAIR_V(K_, W_) \
+    (*reinterpret_cast<const float2 *>(lutb + kVTab + lut_addr<K_>(W_, col)))
     struct PageRegs {
         uint4 kq;
         float nk;
@@ -833,15 +835,15 @@ decode_stream_kernel(SplitParams p) {
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             if constexpr (L == 16)
-                r.vw[k] = lds_b32(smem + so, oV[k]);
+                r.vw[k] = lds_b32(smem + so + k * S, oV);
             else
-                r.vw[k] = *reinterpret_cast<const uint16_t *>(smem + so + oV[k]);
+                r.vw[k] = *reinterpret_cast<const uint16_t *>(smem + so + k * S + oV);
             if constexpr (SQK) {
-                const float2 kv = *reinterpret_cast<const float2 *>(smem + so + oNV[k] - 4);
+                const float2 kv = *reinterpret_cast<const float2 *>(smem + so + k * S + oNV - 4);
                 r.nki[k] = kv.x;
                 r.nv[k] = kv.y;
             } else {
-                r.nv[k] = __uint_as_float(lds_b32(smem + so, oNV[k]));
+                r.nv[k] = __uint_as_float(lds_b32(smem + so + k * S, oNV));
             }
         }
     };
@@ -921,10 +923,10 @@ decode_stream_kernel(SplitParams p) {
         uint32_t ev[4], od[4];
         float2 vc[32];
 #define CDA_V_TILE(K_, SRC_, J_)                                               \
-    vc[4 * (J_) + 0] = CDA_PAIR(K_, SRC_[0]);                                  \
-    vc[4 * (J_) + 1] = CDA_PAIR(K_, SRC_[1]);                                  \
-    vc[4 * (J_) + 2] = CDA_PAIR(K_, SRC_[2]);                                  \
-    vc[4 * (J_) + 3] = CDA_PAIR(K_, SRC_[3]);
+    vc[4 * (J_) + 0] = CDA_PAIR_V(K_, SRC_[0]);                                  \
+    vc[4 * (J_) + 1] = CDA_PAIR_V(K_, SRC_[1]);                                  \
+    vc[4 * (J_) + 2] = CDA_PAIR_V(K_, SRC_[2]);                                  \
+    vc[4 * (J_) + 3] = CDA_PAIR_V(K_, SRC_[3]);
         if constexpr (L == 16) {
 #pragma unroll
             for (int m2 = 0; m2 < 2; ++m2) {
@@ -963,7 +965,7 @@ decode_stream_kernel(SplitParams p) {
             uint32_t qa[4], qbw[4];
             quads(ra, qa);
             quads(rb, qbw);
-#define CDA_QUAD(K_, W_) (*reinterpret_cast<const float4 *>(lutb + lut_addr<K_>(W_, col)))
+#define CDA_QUAD(K_, W_) (*reinterpret_cast<const float4 *>(lutb + kVTab + lut_addr<K_>(W_, col)))
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 // dim j: word j & 3, byte 0 for j < 4, byte 1 otherwise
@@ -1143,6 +1145,7 @@ decode_stream_kernel(SplitParams p) {
         pv_pair(pa1, r[2], r[3]);
     };
 #undef CDA_PAIR
+#undef CDA_PAIR_V
 
     const int nchunks = (wnpages + 3) >> 2;
     const int nfull = (wend - wstart) >> 6;
@@ -1531,6 +1534,14 @@ void fused_plan(int B, int H_kv, int max_seq_len, int *wave_tokens, int *n_split
     *n_splits = (n + wg - 1) / wg;
 }
 
+template <int GS, int L>
+void launch_fused(const SplitParams &p, dim3 grid, hipStream_t st) {
+    if (p.cb_k == p.cb_v)
+        decode_stream_kernel<GS, L, false, true, false><<<grid, kThreads, 0, st>>>(p);
+    else
+        decode_stream_kernel<GS, L, false, true, true><<<grid, kThreads, 0, st>>>(p);
+}
+
 }  // namespace
 
 }  // namespace cda
@@ -1649,8 +1660,9 @@ int decode_impl(const void *q, const void *kv_cache, int slot_bytes, int H_kv,
                         "144-byte slots, 8 KV heads, splits of at most 16384 tokens");
     // Single launch: one workgroup per (sequence, split, KV head) rotates q,
     // streams, merges its waves and (one split per sequence) writes out; more
-    // splits add the combine launch.  Taken with one codebook pointer and the
-    // library's split plan (tile_n 0, or the plan's own tile_n, which the
+    // splits add the combine launch.  Taken for K4V4 and K2V2 caches of any
+    // head count and 16-byte-multiple slot, one codebook pointer or two, with
+    // the library's split plan (tile_n 0, or the plan's own tile_n, which the
     // reference-shaped wrapper passes).
     int plan_tn = 0;
     cda_decode_plan(B, H_q, H_kv, max_seq_len, 0, &plan_tn, nullptr);
@@ -1660,7 +1672,10 @@ int decode_impl(const void *q, const void *kv_cache, int slot_bytes, int H_kv,
     // The single-launch plan never has more splits than the three-launch one
     // (tests pin this over a sweep of shapes); were it to, the three launches
     // below run instead of failing the call.
-    if (stream_shape && !uniform_qk && cb_k == cb_v && (tile_n == 0 || tile_n == plan_tn) &&
+    const bool fused_shape = levels_k == levels_v && slot_bytes % 16 == 0 &&
+                             slot_bytes >= (levels_k == 16 ? 144 : 80) &&
+                             g_allow_stream.load(std::memory_order_relaxed);
+    if (fused_shape && !uniform_qk && (tile_n == 0 || tile_n == plan_tn) &&
         g_allow_fused.load(std::memory_order_relaxed) && nsf <= ns && wf.total <= w.total) {
         SplitParams p{};
         p.q_rot = nullptr;
@@ -1692,14 +1707,14 @@ int decode_impl(const void *q, const void *kv_cache, int slot_bytes, int H_kv,
             return fail(CDA_E_HIP, f + ": hipEventRecord(start) failed");
         if (levels_k == 16) {
             if (group_size == 4)
-                decode_stream_kernel<4, 16, false, true><<<grid, kThreads, 0, st>>>(p);
+                launch_fused<4, 16>(p, grid, st);
             else
-                decode_stream_kernel<8, 16, false, true><<<grid, kThreads, 0, st>>>(p);
+                launch_fused<8, 16>(p, grid, st);
         } else {
             if (group_size == 4)
-                decode_stream_kernel<4, 4, false, true><<<grid, kThreads, 0, st>>>(p);
+                launch_fused<4, 4>(p, grid, st);
             else
-                decode_stream_kernel<8, 4, false, true><<<grid, kThreads, 0, st>>>(p);
+                launch_fused<8, 4>(p, grid, st);
         }
         CDA_LAUNCH_CHECK("decode_stream_kernel");
         if (g_split_stop && hipEventRecord(g_split_stop, st) != hipSuccess)

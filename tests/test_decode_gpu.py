@@ -405,3 +405,39 @@ def test_decode_single_launch_two_rounds(gpu):
     assert _native.decode_fused_plan(64, 8, max(seq))[1] == 1
     case = make_decode_case(7400, seq, H_kv=8, gs=4, fill=0xFF)
     check(run_gpu_decode(case, gpu, gs=4), case.expected)
+
+
+@pytest.mark.parametrize("name,seq_lens,H_kv,gs,levels,slot,two", [
+    ("one_head_wide", [4097, 15], 1, 8, 16, 512, False),
+    ("two_heads_two_cb", [63, 2500, 1], 2, 4, 16, 144, True),
+    ("three_heads_single_split", [513] * 86, 3, 4, 16, 160, False),
+    ("eight_heads_wide_two_cb", [700, 1023], 8, 8, 16, 512, True),
+    ("sixteen_heads", [17, 1111], 16, 4, 16, 144, False),
+    ("k2v2_five_heads_wide", [1500, 65], 5, 4, 4, 96, False),
+    ("k2v2_two_cb", [2047, 3], 8, 4, 4, 80, True),
+    ("k2v2_one_head_two_cb", [640], 1, 8, 4, 80, True),
+])
+def test_decode_single_launch_any_heads_and_slots(gpu, codebooks, name, seq_lens, H_kv, gs, levels,
+                                                  slot, two):
+    """The single launch over head counts and slot widths other than 8 x 144/80
+    bytes and over two codebooks, against the checker and the general kernel
+    (the cache's pad bytes hold garbage)."""
+    from sub0_amd import _native
+    print(f"[decode-fused] case={name} H_kv={H_kv} slot={slot} two={two}", flush=True)
+    cb = None if levels == 16 else codebooks["lloyd_beta4"].astype(np.float32)
+    # The V table keeps the Lloyd table's scale: with a uniform 4-level one the
+    # outputs of a 3-token sequence exceed 4, where one fp16 step (2^-8) is
+    # already more than the tolerance.
+    cbv = ((codebooks[f"lloyd_beta{levels}"] * 0.9).astype(np.float32)) if two else None
+    case = make_decode_case(7500 + len(name), seq_lens, H_kv=H_kv, gs=gs, cb=cb, cb_v=cbv,
+                            fill=0xFF)
+    pad = slot - case.cache.shape[-1]
+    case.cache = np.pad(case.cache, ((0, 0), (0, 0), (0, pad)), constant_values=0xFF)
+    fused = run_gpu_decode(case, gpu, gs=gs)
+    _native.set_stream_kernel(False)
+    try:
+        general = run_gpu_decode(case, gpu, gs=gs)
+    finally:
+        _native.set_stream_kernel(True)
+    check(fused, case.expected)
+    check(fused, general, tol=1e-3)
