@@ -156,17 +156,19 @@ int cda_decode_full_hmma_v3_noalloc(const void *q, const void *kv_cache, int64_t
 int cda_decode_set_timing_events(void *start_event, void *stop_event);
 
 /* Selects the decode split kernel for later calls (process-wide; default 1).
- * enable=1 lets cda_decode_full_hmma_v3 use the page-streaming kernel when the
- * cache is 8 KV heads x 144-byte (K4V4) or 80-byte (K2V2) slots and the K and
- * V codebooks hold equal bits (one pointer, or two compared on the device);
- * enable=0 always takes the general kernel.  Both produce the same result to
+ * enable=1 lets cda_decode_full_hmma_v3 use the page-streaming kernel: in its
+ * single-launch form (below) for K4V4 and K2V2 caches of any head count and any
+ * slot width of a multiple of 16 bytes, with one codebook or two; in its
+ * three-launch form for 8 KV heads x 144-byte (K4V4) or 80-byte (K2V2) slots
+ * when the K and V codebooks hold equal bits (one pointer, or two compared on
+ * the device).  enable=0 always takes the general kernel.  Both produce the same result to
  * fp32 rounding of the softmax sums.  No reference counterpart: the reference
  * has one decode kernel; this exists for A/B measurement and tests. */
 int cda_decode_set_stream_kernel(int enable);
 
 /* Selects the single-launch decode for later calls (process-wide; default 1).
  * enable=1 lets cda_decode_full_hmma_v3 run, where the page-streaming kernel
- * applies with one codebook pointer for K and V and the library's split plan
+ * applies, with one codebook pointer or two and the library's split plan
  * (tile_n = 0, or the tile_n that cda_decode_plan returns for tile_n = 0, which
  * is what the reference-shaped wrapper passes), one kernel per call: each workgroup takes one KV head over a token
  * range, rotates q itself, merges its waves' partials and, when its range is
