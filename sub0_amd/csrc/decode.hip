@@ -92,6 +92,7 @@ struct SplitParams {
     const float *R;             // (128, 128) fp32 rotation
     uint16_t *out;              // (B, H_q, 128) fp16
     int wave_tokens;            // multiple of 64
+    int bs_shift;               // log2(block_size) when it is a power of two, else -1
     int xcd_map;                // 1: the heads of a (sequence, split) share an XCD
 };
 
@@ -637,9 +638,37 @@ decode_stream_kernel(SplitParams p) {
         h = wave;
     }
 
+    const int bs = p.block_size;
+    const int start = sp * p.tile_n;
+    // Cache block of token t (FUSED: a shift for the usual block sizes).
+    auto block_of = [&](int t) CDA_INLINE {
+        return FUSED && p.bs_shift >= 0 ? t >> p.bs_shift : t / bs;
+    };
+    // FUSED: every load of the prologue that does not need the sequence length
+    // goes out first, so their latencies overlap: the rows of the wave's first
+    // four pages (lane k: page k; the index is clamped to the table row, an
+    // entry past the sequence is not used), the codebook, q of the head's GQA
+    // group and this wave's 16 columns of R.
+    constexpr int kQPer = GS * kD / kThreads;             // q values per thread
+    int first_row = 0;
+    float cb_lane = 0.0f, rcol[FUSED ? kD / 4 : 1];
+    uint16_t qv[FUSED ? kQPer : 1];
+    if constexpr (FUSED) {
+        const int32_t *bt = p.block_table + (int64_t)b * p.bt_stride;
+        const int t0 = start + wave * p.wave_tokens + 16 * (lane & 3);
+        const int blk = block_of(t0);
+        first_row = bt[min(blk, p.bt_stride - 1)] * bs + (t0 - blk * bs);
+#pragma unroll
+        for (int i = 0; i < kQPer; ++i)
+            qv[i] = p.q[((int64_t)b * p.H_q + (int64_t)h * GS) * kD + tid + i * kThreads];
+#pragma unroll
+        for (int m = 0; m < kD / 4; ++m)
+            rcol[m] = p.R[(4 * m + q4) * kD + 16 * wave + r16];
+    }
+    if (lane < L) cb_lane = SQK ? p.cb_v[lane] : p.cb_k[lane];
+    if (TWO && lane >= 16 && lane < 16 + L) cb_lane = p.cb_v[lane - 16];
     const int seq_len =
         __builtin_amdgcn_readfirstlane(min(p.seq_lens[b], p.bt_stride * p.block_size));
-    const int start = sp * p.tile_n;
     const int end = min(start + p.tile_n, seq_len);
     const int64_t part_row = ((int64_t)b * p.n_splits + sp) * p.H_q + (int64_t)h * GS;
     // This wave's token range: the whole split, or (FUSED) its own share.
@@ -682,20 +711,12 @@ decode_stream_kernel(SplitParams p) {
         src[i] = (uint32_t)((piece / kPieces) * row_bytes + (piece % kPieces) * 16);
     }
 
-    const int bs = p.block_size;
     const int npages = (end - start + 15) >> 4;          // the workgroup's pages
     const int wpage0 = (wstart - start) >> 4;            // this wave's first among them
     const int wnpages = (wend - wstart + 15) >> 4;
     const uint32_t ring_w = __builtin_amdgcn_readfirstlane(lds_u32addr(smem)) + kStreamRingOff +
                             wave * (kStreamPages * kHP);
     int32_t *page_row = reinterpret_cast<int32_t *>(smem + kStreamPidOff);
-    {
-        const int32_t *bt = p.block_table + (int64_t)b * p.bt_stride;
-        for (int t = tid; t < npages; t += kThreads) {
-            const int t0 = start + 16 * t;
-            page_row[t] = bt[t0 / bs] * bs + (t0 % bs);
-        }
-    }
     const uint8_t *kv_h = p.kv + (int64_t)h * p.slot_bytes;
     const uint32_t page_bytes = (uint32_t)(16 * row_bytes - h * p.slot_bytes);
     // DMA of the page starting at cache row row0 into ring slot k.
@@ -713,24 +734,29 @@ decode_stream_kernel(SplitParams p) {
     auto issue = [&](int t, int k) CDA_INLINE {
         issue_row(__builtin_amdgcn_readfirstlane(page_row[wpage0 + t]), k);
     };
-    // The first chunk's pages straight from the block table (wave-uniform
-    // loads), before the tables are built: their latency overlaps the set-up.
-    {
-        const int32_t *bt = p.block_table + (int64_t)b * p.bt_stride;
+    // Cache row of the workgroup's page t.
+    auto row_of = [&](int t) CDA_INLINE {
+        const int t0 = start + 16 * t, blk = block_of(t0);
+        return p.block_table[(int64_t)b * p.bt_stride + blk] * bs + (t0 - blk * bs);
+    };
+    uint4 qb[4];
+    // The first chunk's pages go out before the tables are built, so their
+    // latency overlaps the set-up.
+    if constexpr (FUSED) {
+        // The loads above are waited for first: the DMAs are outside the
+        // compiler's count of loads in flight, and behind them every wait of
+        // its own would also wait for the pages.
+#pragma unroll
+        for (int m = 0; m < kD / 4; ++m) asm volatile("" : "+v"(rcol[m]));
 #pragma unroll
         for (int k = 0; k < kStreamPages; ++k)
-            if (k < wnpages) {
-                const int t0 = wstart + 16 * k;
-                issue_row((int64_t)__builtin_amdgcn_readfirstlane(bt[t0 / bs]) * bs + t0 % bs, k);
-            }
-    }
-    uint4 qb[4];
-    if constexpr (FUSED) {
-        // q of this head's GQA group as fp32, for the rotation below.
-        float *qs = reinterpret_cast<float *>(smem + kFusedQOff);
-        const uint16_t *qg = p.q + ((int64_t)b * p.H_q + (int64_t)h * GS) * kD;
-        for (int i = tid; i < GS * kD; i += kThreads) qs[i] = h2f(qg[i]);
+            if (k < wnpages) issue_row(__builtin_amdgcn_readlane(first_row, k), k);
     } else {
+#pragma unroll
+        for (int k = 0; k < kStreamPages; ++k)
+            if (k < wnpages)
+                issue_row(__builtin_amdgcn_readfirstlane(row_of(wpage0 + k)), k);
+        for (int t = tid; t < npages; t += kThreads) page_row[t] = row_of(t);
         const uint16_t *qg =
             p.q_rot + ((int64_t)b * p.H_q + (int64_t)h * GS + (r16 & (GS - 1))) * kD + 32 * q4;
 #pragma unroll
@@ -750,44 +776,77 @@ decode_stream_kernel(SplitParams p) {
         a += __shfl_xor(a, 32);
         qsum_neg = -0.9375f * a;
     }
-    {
-        // The codebook goes through LDS first: a global load per table entry
-        // would put 32 dependent memory round trips in every thread's
-        // prologue.
-        __shared__ float cbs[TWO ? 32 : 16];
-        if (tid < L) cbs[tid] = SQK ? p.cb_v[tid] : p.cb_k[tid];
-        if (TWO && tid >= 16 && tid < 16 + L) cbs[tid] = p.cb_v[tid - 16];
-        __syncthreads();
-        uint32_t *lut = reinterpret_cast<uint32_t *>(smem);
-        for (int i = tid; i < kLut2Bytes / 4; i += kThreads) {
-            const int e = i >> 6;
-            const float *cb = cbs + (TWO ? (i & 32) >> 1 : 0);   // second half of a row: V
-            if constexpr (L == 16)
-                lut[i] = __float_as_uint(cb[(i & 1) ? (e & 15) : (e >> 4)]);
-            else   // quad q of row e: the code in bits 7-2q:6-2q (dims 4j + q)
-                lut[i] = __float_as_uint(cb[(e >> (6 - 2 * (i & 3))) & 3]);
+    int rows[FUSED ? kFusedMaxPages / kThreads : 1];
+    if constexpr (FUSED) {
+        // q as fp32, element k = 4m + i of a row at 32i + m: the order in which
+        // the lanes of the rotation below take it.
+        float *qs = reinterpret_cast<float *>(smem + kFusedQOff);
+#pragma unroll
+        for (int i = 0; i < kQPer; ++i) {
+            const int o = tid + i * kThreads, k = o & (kD - 1);
+            qs[(o & ~(kD - 1)) + (k & 3) * 32 + (k >> 2)] = h2f(qv[i]);
+        }
+        // Page rows of the later chunks; stored after the rotation.
+#pragma unroll
+        for (int i = 0; i < kFusedMaxPages / kThreads; ++i) {
+            rows[i] = 0;
+            if (tid + i * kThreads < npages) rows[i] = row_of(tid + i * kThreads);
         }
     }
-    if constexpr (FUSED) {
-        // q_rot = fp16(q @ R): the fp32 fma chain over k in ascending order,
-        // as rotate_q_kernel computes it (compression.py:290-291).
-        const float *qs = reinterpret_cast<const float *>(smem + kFusedQOff);
-        uint16_t *qr = reinterpret_cast<uint16_t *>(smem + kFusedQrOff);
-        for (int o = tid; o < GS * kD; o += kThreads) {
-            const float *qrow = qs + (o >> 7) * kD;
-            const float *rc = p.R + (o & (kD - 1));
-            float a = 0.0f;
-#pragma unroll 16
-            for (int k = 0; k < kD; ++k) a = fmaf(qrow[k], rc[k * kD], a);
-            qr[o] = f2h_after_f32(a);
+    {
+        // Dequant table: 16 lanes write one 256-byte row, the entries taken
+        // from the codebook held one level per lane.
+        const int half = TWO && r16 >= 8 ? 16 : 0;             // second half of a row: V
+#pragma unroll
+        for (int i = 0; i < 256 / (4 * kWaves); ++i) {
+            const int e = 4 * (wave + kWaves * i) + q4;
+            float4 v;
+            if constexpr (L == 16) {
+                v.x = v.z = __shfl(cb_lane, half + (e >> 4));
+                v.y = v.w = __shfl(cb_lane, half + (e & 15));
+            } else {   // the code in bits 7:6 first (dims 4j .. 4j + 3)
+                v = make_float4(__shfl(cb_lane, half + (e >> 6)),
+                                __shfl(cb_lane, half + ((e >> 4) & 3)),
+                                __shfl(cb_lane, half + ((e >> 2) & 3)),
+                                __shfl(cb_lane, half + (e & 3)));
+            }
+            reinterpret_cast<float4 *>(smem)[16 * e + r16] = v;
         }
     }
     __syncthreads();
     if constexpr (FUSED) {
-        const uint16_t *qr = reinterpret_cast<const uint16_t *>(smem + kFusedQrOff) +
-                             (r16 & (GS - 1)) * kD + 32 * q4;
+        // q_rot = fp16(q @ R) (compression.py:290-291), sixteen columns per
+        // wave: v_mfma_f32_16x16x4_f32 adds its four products to the
+        // accumulator one after the other with one rounding each, so the 32 of
+        // them are the fp32 fma chain over ascending k that rotate_q_kernel and
+        // the checker compute, bit for bit.  R is read once per workgroup
+        // (64 KB), where a thread per output read it once per query head: 1.85
+        // us of the kernel, 3.8 us with 8 queries per head.  With the loads
+        // above in one batch and the table written in 16-byte pieces (2.1 us
+        // with four), a call takes 17.9 -> 15.8 us at B=1, N=4K and 33.0 ->
+        // 28.4 us for 16 sequences of 4K-16K tokens, 2 KV heads x 8 queries.
+        const float4 *qa = reinterpret_cast<const float4 *>(smem + kFusedQOff) +
+                           ((r16 & (GS - 1)) * kD + q4 * 32) / 4;
+        floatx4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int s = 0; s < 4; ++s) qb[s] = *reinterpret_cast<const uint4 *>(qr + 8 * s);
+        for (int m4 = 0; m4 < kD / 16; ++m4) {
+            const float4 a = qa[m4];
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, rcol[4 * m4 + 0], acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, rcol[4 * m4 + 1], acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, rcol[4 * m4 + 2], acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, rcol[4 * m4 + 3], acc, 0, 0, 0);
+        }
+        uint16_t *qr = reinterpret_cast<uint16_t *>(smem + kFusedQrOff);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (4 * q4 + i < GS) qr[(4 * q4 + i) * kD + 16 * wave + r16] = f2h_after_f32(acc[i]);
+#pragma unroll
+        for (int i = 0; i < kFusedMaxPages / kThreads; ++i)
+            if (tid + i * kThreads < npages) page_row[tid + i * kThreads] = rows[i];
+        __syncthreads();
+        const uint16_t *qw = qr + (r16 & (GS - 1)) * kD + 32 * q4;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) qb[s] = *reinterpret_cast<const uint4 *>(qw + 8 * s);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
@@ -1705,6 +1764,7 @@ int decode_impl(const void *q, const void *kv_cache, int slot_bytes, int H_kv,
         p.R = rot_f32;
         p.out = static_cast<uint16_t *>(out);
         p.wave_tokens = wave_tokens;
+        p.bs_shift = (block_size & (block_size - 1)) == 0 ? __builtin_ctz(block_size) : -1;
         const int units = B * nsf;
         p.xcd_map = (units % 8 == 0) ? 1 : 0;
         const dim3 grid(units * H_kv);
