@@ -1379,152 +1379,146 @@ __device__ __forceinline__ float wave_sum(float v) {
 
 // Merge split partials (attention.py:239-272: m* = max m_i, weights
 // exp(m_i - m*), empty splits weigh 0, l clamped at 1e-30), round O_rot to
-// fp16 and unrotate: out[j] = sum_k fp16(O_rot)[k] * R[j][k].  One 256-thread
-// block per (4 q-heads, sequence): wave w merges head w (two splits per wave
-// instruction, four dims per lane, 32 splits' loads in flight at a time).  R is staged in LDS in its own row
-// order with rows padded to 132 floats, so the global reads are coalesced,
-// all sixteen per thread are in flight at once, and the epilogue's 16-byte
-// row reads (lane j reads row j) fall in distinct banks.
-constexpr int kRPad = kD + 4;
-
+// fp16 and unrotate: out[j] = sum_k fp16(O_rot)[k] * R[j][k], fp32.
+//
 // HPB heads per 256-thread block: 4 (one wave per head) when the grid fills
 // the chip, else 1 (the four waves take interleaved 32-split batches of one
-// head and their partial sums are added in a fixed order).
+// head and their partial sums are added in a fixed order).  Lanes 0-31 of a
+// wave take the even splits and lanes 32-63 the odd ones, four dims per lane.
+//
+// The kernel is a chain of latencies, so all its loads go out at the start: the
+// first 32 splits' partials do not wait for the weights, and R goes straight
+// into registers, 32 lanes per row (thread t: rows (t >> 5) + 8u, columns 4 *
+// (t & 31) ..), which makes the product 64 fmas per thread and head and a
+// 32-lane reduction.  Against R staged in LDS for one wave to walk its rows, a
+// call with several splits takes 1.2-1.4 us less (B=1: N=4K 15.9 -> 14.6 us,
+// N=64K 27.8 -> 26.5).
 template <int HPB>
 __global__ void __launch_bounds__(256)
 combine_kernel(const float *part_o, const float *part_ml, const float *R, uint16_t *out,
                int H_q, int n_splits) {
     static_assert(HPB == 4 || HPB == 1, "heads per block");
     constexpr int kWph = 4 / HPB;                  // waves per head
-    __shared__ __align__(16) float Rs[kD * kRPad];
+    constexpr int kRows = kD / 8;                  // rows of R per thread
     __shared__ float wts[4][kMaxSplits];
-    __shared__ __align__(16) float orot[4][kD];
+    __shared__ __align__(16) float osum[4][kD];
+    __shared__ float lsum[4];
     const int b = blockIdx.y, t = threadIdx.x;
     const int h0 = blockIdx.x * HPB;
-    const int hh = (HPB == 4) ? (t >> 6) : 0, lane = t & 63;
-    const int wsub = (HPB == 4) ? 0 : (t >> 6);   // this wave's share of the splits
-    const int wslot = t >> 6;                      // this wave's rows of wts / orot
-    const int h = h0 + hh;
-    float4 rr[kD * kD / 4 / 256];
+    const int wave = t >> 6, lane = t & 63;
+    const int wsub = (HPB == 4) ? 0 : wave;        // this wave's share of the splits
+    const int h = h0 + ((HPB == 4) ? wave : 0);
+    const int half = lane >> 5, d4 = 4 * (lane & 31);
+    const bool live = h < H_q;
+    const int64_t base = (int64_t)b * n_splits * H_q + h;
+    const float *po = part_o + base * kD + d4;
+    const int64_t step = (int64_t)H_q * kD;
+    // Empty splits store zeros, so every partial is read unconditionally.
+    float4 v[16];
+    auto load_batch = [&](int s0) CDA_INLINE {
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+            const int s = s0 + 2 * u + half;
+            v[u] = (live && s < n_splits)
+                       ? *reinterpret_cast<const float4 *>(po + (int64_t)s * step)
+                       : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+    };
+    // All (m, l) pairs of this head in flight at once (up to kMaxSplits).
+    constexpr int kPer = kMaxSplits / 64;
+    float2 ml[kPer];
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+        const int s = lane + 64 * i;
+        ml[i] = (live && s < n_splits)
+                    ? *reinterpret_cast<const float2 *>(part_ml + (base + (int64_t)s * H_q) * 2)
+                    : make_float2(-INFINITY, 0.0f);
+    }
+    load_batch(32 * wsub);
+    float4 rr[kRows];
     {
         const float4 *R4 = reinterpret_cast<const float4 *>(R);
 #pragma unroll
-        for (int u = 0; u < kD * kD / 4 / 256; ++u) rr[u] = R4[t + 256 * u];
+        for (int u = 0; u < kRows; ++u) rr[u] = R4[t + 256 * u];
     }
-    const bool live = h < H_q;
-    const int64_t base = (int64_t)b * n_splits * H_q + h;
-    float L = 0.0f;
-    if (live) {
-        // All (m, l) pairs of this head in flight at once (up to kMaxSplits).
-        constexpr int kPer = kMaxSplits / 64;
-        float2 ml[kPer];
+    float mx = -INFINITY;
 #pragma unroll
-        for (int i = 0; i < kPer; ++i) {
-            const int s = lane + 64 * i;
-            ml[i] = (s < n_splits)
-                        ? *reinterpret_cast<const float2 *>(part_ml + (base + (int64_t)s * H_q) * 2)
-                        : make_float2(-INFINITY, 0.0f);
+    for (int i = 0; i < kPer; ++i) mx = fmaxf(mx, ml[i].x);
+    mx = wave_max(mx);
+    float lp = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+        if (64 * i >= n_splits) break;
+        const float w = (ml[i].x == -INFINITY) ? 0.0f : exp2f(ml[i].x - mx);
+        wts[wave][lane + 64 * i] = w;
+        if (w != 0.0f) lp += w * ml[i].y;
+    }
+    lp = wave_sum(lp);
+    if (lane == 0) lsum[wave] = lp;
+    __builtin_amdgcn_wave_barrier();
+    float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int s0 = 32 * wsub; s0 < n_splits; s0 += 32 * kWph) {
+        if (s0 != 32 * wsub) load_batch(s0);
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+            const int s = s0 + 2 * u + half;
+            const float w = (s < n_splits) ? wts[wave][s] : 0.0f;
+            o.x = fmaf(w, v[u].x, o.x);
+            o.y = fmaf(w, v[u].y, o.y);
+            o.z = fmaf(w, v[u].z, o.z);
+            o.w = fmaf(w, v[u].w, o.w);
         }
-        float mx = -INFINITY;
-#pragma unroll
-        for (int i = 0; i < kPer; ++i) mx = fmaxf(mx, ml[i].x);
-        mx = wave_max(mx);
-        float lp = 0.0f;
-#pragma unroll
-        for (int i = 0; i < kPer; ++i) {
-            const int s = lane + 64 * i;
-            const float w = (ml[i].x == -INFINITY) ? 0.0f : exp2f(ml[i].x - mx);
-            if (s < n_splits) wts[wslot][s] = w;
-            if (w != 0.0f) lp += w * ml[i].y;
-        }
-        L = wave_sum(lp);
     }
-#pragma unroll
-    for (int u = 0; u < kD * kD / 4 / 256; ++u) {
-        const int i = t + 256 * u;
-        *reinterpret_cast<float4 *>(Rs + (i >> 5) * kRPad + 4 * (i & 31)) = rr[u];
-    }
+    auto sum_halves = [](float x) {
+        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x),
+                                                        false, false);
+        return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    };
+    o = make_float4(sum_halves(o.x), sum_halves(o.y), sum_halves(o.z), sum_halves(o.w));
+    if (half == 0) *reinterpret_cast<float4 *>(&osum[wave][d4]) = o;
     __syncthreads();
-    if (live) {
-        // Empty splits store zeros, so every partial is read unconditionally.
-        // Lanes 0-31 take the even splits and lanes 32-63 the odd ones, four
-        // dims per lane, sixteen 16-byte loads in flight: 32 splits per batch.
-        const int half = lane >> 5, d4 = 4 * (lane & 31);
-        const float *po = part_o + base * kD + d4;
-        const int64_t step = (int64_t)H_q * kD;
-        float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
-        for (int s0 = 32 * wsub; s0 < n_splits; s0 += 32 * kWph) {
-            float4 v[16];
 #pragma unroll
-            for (int u = 0; u < 16; ++u) {
-                const int s = s0 + 2 * u + half;
-                v[u] = (s < n_splits) ? *reinterpret_cast<const float4 *>(po + (int64_t)s * step)
-                                      : make_float4(0.f, 0.f, 0.f, 0.f);
-            }
+    for (int hh = 0; hh < HPB; ++hh) {
+        if (h0 + hh >= H_q) break;
+        // O_rot of dims d4 .. d4 + 3: the head's sums (its four waves' in a
+        // fixed order), normalised and rounded to fp16.
+        float4 x = *reinterpret_cast<const float4 *>(&osum[hh][d4]);
+        if constexpr (HPB == 1) {
 #pragma unroll
-            for (int u = 0; u < 16; ++u) {
-                const int s = s0 + 2 * u + half;
-                const float w = (s < n_splits) ? wts[wslot][s] : 0.0f;
-                o.x = fmaf(w, v[u].x, o.x);
-                o.y = fmaf(w, v[u].y, o.y);
-                o.z = fmaf(w, v[u].z, o.z);
-                o.w = fmaf(w, v[u].w, o.w);
+            for (int w = 1; w < 4; ++w) {
+                const float4 y = *reinterpret_cast<const float4 *>(&osum[w][d4]);
+                x = make_float4(x.x + y.x, x.y + y.y, x.z + y.z, x.w + y.w);
             }
         }
-        auto sum_halves = [](float x) {
-            const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x),
-                                                            false, false);
-            return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-        };
-        o.x = sum_halves(o.x);
-        o.y = sum_halves(o.y);
-        o.z = sum_halves(o.z);
-        o.w = sum_halves(o.w);
-        const float inv = 1.0f / fmaxf(L, 1e-30f);
-        if (HPB == 4 && half == 0) {
-            orot[hh][d4 + 0] = h2f(f2h_after_f32(o.x * inv));
-            orot[hh][d4 + 1] = h2f(f2h_after_f32(o.y * inv));
-            orot[hh][d4 + 2] = h2f(f2h_after_f32(o.z * inv));
-            orot[hh][d4 + 3] = h2f(f2h_after_f32(o.w * inv));
-        }
-        if (HPB == 1 && half == 0)
-            *reinterpret_cast<float4 *>(&orot[wsub][d4]) = make_float4(o.x, o.y, o.z, o.w);
+        const float inv = 1.0f / fmaxf(lsum[hh], 1e-30f);
+        x.x = h2f(f2h_after_f32(x.x * inv));
+        x.y = h2f(f2h_after_f32(x.y * inv));
+        x.z = h2f(f2h_after_f32(x.z * inv));
+        x.w = h2f(f2h_after_f32(x.w * inv));
+        float a[kRows];
+#pragma unroll
+        for (int u = 0; u < kRows; ++u)
+            a[u] = fmaf(x.w, rr[u].w, fmaf(x.z, rr[u].z, fmaf(x.y, rr[u].y, x.x * rr[u].x)));
+        // Sum the sixteen rows over the 32 lanes: at each step a lane keeps the
+        // half of its rows that its own lane bit names, so four steps leave
+        // one row per lane pair, row u = lane bits 4..1.
+#define CDA_HALVE(N_, M_)                                                                        \
+    _Pragma("unroll") for (int u = 0; u < (N_); ++u) {                                           \
+        const bool up = (lane & (M_)) != 0;                                                      \
+        const float keep = up ? a[u + (N_)] : a[u], send = up ? a[u] : a[u + (N_)];              \
+        a[u] = keep + __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(send),           \
+                                                                 0x1F | ((M_) << 10)));          \
     }
-    __syncthreads();
-    if (!live || wsub != 0) return;
-    if (HPB == 1) {
-        // Wave 0: add the four waves' partial sums (fixed order), normalise,
-        // round O_rot to fp16.
-        const float inv = 1.0f / fmaxf(L, 1e-30f);
-        const float s0 = ((orot[0][lane] + orot[1][lane]) + orot[2][lane]) + orot[3][lane];
-        const float s1 = ((orot[0][lane + 64] + orot[1][lane + 64]) + orot[2][lane + 64]) +
-                         orot[3][lane + 64];
-        // Every lane has read all four rows before row 0 is overwritten.
-        __builtin_amdgcn_wave_barrier();
-        orot[0][lane] = h2f(f2h_after_f32(s0 * inv));
-        orot[0][lane + 64] = h2f(f2h_after_f32(s1 * inv));
-        __builtin_amdgcn_wave_barrier();
+        CDA_HALVE(8, 16)
+        CDA_HALVE(4, 8)
+        CDA_HALVE(2, 4)
+        CDA_HALVE(1, 2)
+#undef CDA_HALVE
+        a[0] += __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(a[0]), 0x1F | (1 << 10)));
+        if (!(lane & 1))
+            out[((int64_t)b * H_q + h0 + hh) * kD + (t >> 5) + 8 * ((lane >> 1) & 15)] =
+                f2h_after_f32(a[0]);
     }
-    const float *r0 = Rs + lane * kRPad;
-    const float *r1 = Rs + (lane + 64) * kRPad;
-    float a0 = 0.0f, a1 = 0.0f;
-#pragma unroll 8
-    for (int k = 0; k < kD; k += 4) {
-        const float4 o = *reinterpret_cast<const float4 *>(&orot[hh][k]);
-        const float4 x = *reinterpret_cast<const float4 *>(r0 + k);
-        const float4 y = *reinterpret_cast<const float4 *>(r1 + k);
-        a0 = fmaf(o.x, x.x, a0);
-        a0 = fmaf(o.y, x.y, a0);
-        a0 = fmaf(o.z, x.z, a0);
-        a0 = fmaf(o.w, x.w, a0);
-        a1 = fmaf(o.x, y.x, a1);
-        a1 = fmaf(o.y, y.y, a1);
-        a1 = fmaf(o.z, y.z, a1);
-        a1 = fmaf(o.w, y.w, a1);
-    }
-    const int64_t row = ((int64_t)b * H_q + h) * kD;
-    out[row + lane] = f2h_after_f32(a0);
-    out[row + lane + 64] = f2h_after_f32(a1);
 }
 
 struct WsLayout {
