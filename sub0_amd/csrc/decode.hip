@@ -1495,6 +1495,9 @@ combine_kernel(const float *part_o, const float *part_ml, const float *R, uint16
         x.y = h2f(f2h_after_f32(x.y * inv));
         x.z = h2f(f2h_after_f32(x.z * inv));
         x.w = h2f(f2h_after_f32(x.w * inv));
+        // Widened once: left visible, the conversion is folded into every fma
+        // (v_fma_mix_f32, about twice the issue cost of v_fma_f32).
+        asm volatile("" : "+v"(x.x), "+v"(x.y), "+v"(x.z), "+v"(x.w));
         float a[kRows];
 #pragma unroll
         for (int u = 0; u < kRows; ++u)
