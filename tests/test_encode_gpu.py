@@ -166,3 +166,29 @@ def test_encode_config2_scale_k2v2(gpu, codebooks):
     exp = expected_cache(k, v, slots, cb, num_slots, 80, 0)
     got = run_gpu_encode(gpu, k, v, slots, cb, num_slots, 80, 0)
     assert np.array_equal(got, exp)
+
+
+@pytest.mark.parametrize("levels,T,H_kv", [
+    (16, 512, 8),      # the last batch of the 16-lane form: 4096 items
+    (16, 513, 8),      # the first of the MFMA form, a part-filled last block
+    (4, 1367, 3),      # 4101 items: five in the last wave
+    (16, 4113, 1),
+])
+def test_encode_mfma_form_edges(gpu, codebooks, levels, T, H_kv):
+    """Batches around the switch between the two encode kernels and with part-
+    filled waves, a codebook for each role, padding tokens: every byte equal."""
+    print(f"[encode] mfma form levels={levels} T={T} H_kv={H_kv}", flush=True)
+    cb_k = codebooks["lloyd_beta16" if levels == 16 else "lloyd_beta4"]
+    cb_v = codebooks["uniform16" if levels == 16 else "uniform4"]
+    k = synth.kv_with_outliers(521, (T, H_kv, 128))
+    v = synth.normal_f16(522, (T, H_kv, 128))
+    k[5] = 0                              # a zero vector: the clamped norm
+    v[7, 0, :3] = (6e-8, -6e-8, 0)        # fp16 subnormals
+    v[7, 0, 3:] = 0
+    slots = synth.permuted_block_table(523, 1, T + 9)[0][:T].astype(np.int64)
+    slots[::13] = -1
+    sb = 144 if levels == 16 else 80
+    exp = expected_cache(k, v, slots, cb_k, T + 9, sb, 0x3C, cb_v=cb_v)
+    got = run_gpu_encode(gpu, k, v, slots, cb_k, T + 9, sb, 0x3C, cb_v=cb_v)
+    bad = np.argwhere(got != exp)
+    assert bad.size == 0, f"{len(bad)} mismatching bytes, first {bad[:5].tolist()}"
