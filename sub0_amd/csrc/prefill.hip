@@ -844,8 +844,12 @@ paged_to_dense_kernel(const uint8_t *kv, int64_t row_bytes, int slot_bytes, int 
 // y = fp16(scale * x H) for rows of 128 fp16 (Sylvester order, natural index):
 // 16 lanes per row, 8 elements per lane; butterflies over index bits 0-2 in
 // registers and bits 3-6 across lanes, in fp32.
+// Two tensors of one shape may go in one launch (blockIdx.y).
 __global__ void __launch_bounds__(256)
-hadamard128_kernel(const uint16_t *x, uint16_t *y, int64_t rows, float scale) {
+hadamard128_kernel(const uint16_t *x0, uint16_t *y0, const uint16_t *x1, uint16_t *y1, int64_t rows,
+                   float scale) {
+    const uint16_t *x = blockIdx.y ? x1 : x0;
+    uint16_t *y = blockIdx.y ? y1 : y0;
     const int64_t row = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
     const int l16 = threadIdx.x & 15;
     float v[8] = {};
@@ -1001,10 +1005,13 @@ int launch_prefill(const PrefillParams &p, int B, int max_q, hipStream_t st, con
 }
 
 // Key-split plan: split only when the unsplit grid leaves CUs idle (fewer
-// than 256 workgroups), into splits of at least 4 key tiles (256 keys), aiming
-// at one round of ~256 workgroups (one per CU: the kernel's LDS admits one);
-// at most kMaxKsplit splits.  Targets of 512 and 1024 workgroups (two and four
-// rounds of shorter splits) measured 5-30 % slower.
+// than 256 workgroups), into splits of at least 4 key tiles (256 keys), at most
+// kMaxKsplit of them.  One workgroup fits a CU, so a grid runs in rounds of 256;
+// the split count is the one with the least rounds x (tiles per split + 3),
+// a workgroup's set-up and epilogue costing about three tiles.  Rounding the
+// count up to fill 256 workgroups put 80 query blocks in 320 workgroups, two
+// rounds of 20 tiles where three splits run one of 27: 2 x 200-300 queries over
+// 5000 keys, hybrid, 146 -> 106 us a call.
 constexpr int kMaxKsplit = 64;
 static_assert(kMaxKsplit <= 64, "prefill_combine_kernel: one lane per split");
 void prefill_ksplit_plan(int B, int H_q, int H_kv, int max_q, int max_k, int *n_split,
@@ -1012,19 +1019,20 @@ void prefill_ksplit_plan(int B, int H_q, int H_kv, int max_q, int max_k, int *n_
     const int qb = 32 * (kWaves / (H_q / H_kv));
     const int64_t wgs = (int64_t)((max_q + qb - 1) / qb) * B * H_kv;
     const int tiles = (max_k + kBN - 1) / kBN;
-    int ns = 1;
-    if (wgs > 0 && wgs < 256) {
-        ns = (int)std::min<int64_t>((256 + wgs - 1) / wgs, tiles / 4);
-        ns = std::min(ns, max_split);
+    *n_split = 1;
+    *split_tiles = tiles;
+    if (wgs <= 0 || wgs >= 256) return;
+    constexpr int kFixed = 3;                              // set-up and epilogue, in tiles
+    int64_t best = tiles + kFixed;
+    for (int s = 2; s <= std::min(tiles / 4, max_split); ++s) {
+        const int per = (tiles + s - 1) / s, ns = (tiles + per - 1) / per;
+        const int64_t cost = (wgs * ns + 255) / 256 * (per + kFixed);
+        if (cost < best) {
+            best = cost;
+            *n_split = ns;
+            *split_tiles = per;
+        }
     }
-    if (ns < 2) {
-        *n_split = 1;
-        *split_tiles = tiles;
-        return;
-    }
-    const int per = (tiles + ns - 1) / ns;
-    *split_tiles = per;
-    *n_split = (tiles + per - 1) / per;
 }
 
 size_t prefill_ws_bytes(int T, int H_q, int n_split) {
@@ -1378,7 +1386,7 @@ extern "C" int cda_hadamard128_fp16(const void *x, void *y, int64_t rows, float 
                 "cda_hadamard128_fp16: x and y must be 16-byte aligned");
     if (rows == 0) return CDA_OK;
     hadamard128_kernel<<<(unsigned)((rows + 15) / 16), 256, 0, static_cast<hipStream_t>(stream)>>>(
-        static_cast<const uint16_t *>(x), static_cast<uint16_t *>(y), rows, scale);
+        static_cast<const uint16_t *>(x), static_cast<uint16_t *>(y), nullptr, nullptr, rows, scale);
     CDA_LAUNCH_CHECK("hadamard128_kernel");
     return CDA_OK;
 }
@@ -1466,12 +1474,10 @@ extern "C" int cda_prefill_hybrid_rawkv(const void *q, const void *k_new, const 
     uint16_t *v_rot = reinterpret_cast<uint16_t *>(ws + h.part_bytes + h.kv_bytes);
     const int64_t kv_rows = (int64_t)T * H_kv;
     const float hs = 0.08838834764831845f;
-    hadamard128_kernel<<<(unsigned)((kv_rows + 15) / 16), 256, 0, st>>>(
-        static_cast<const uint16_t *>(k_new), k_rot, kv_rows, hs);
-    CDA_LAUNCH_CHECK("cda_prefill_hybrid_rawkv: hadamard128_kernel (K)");
-    hadamard128_kernel<<<(unsigned)((kv_rows + 15) / 16), 256, 0, st>>>(
-        static_cast<const uint16_t *>(v_new), v_rot, kv_rows, hs);
-    CDA_LAUNCH_CHECK("cda_prefill_hybrid_rawkv: hadamard128_kernel (V)");
+    hadamard128_kernel<<<dim3((unsigned)((kv_rows + 15) / 16), 2), 256, 0, st>>>(
+        static_cast<const uint16_t *>(k_new), k_rot, static_cast<const uint16_t *>(v_new), v_rot,
+        kv_rows, hs);
+    CDA_LAUNCH_CHECK("cda_prefill_hybrid_rawkv: hadamard128_kernel");
 
     PrefillParams p{};
     p.q = static_cast<const uint16_t *>(q);

@@ -76,6 +76,11 @@ def test_prefill_key_split_plan():
     # 4000 keys = 63 tiles: min(64, 63 // 4) = 15 splits -> 5 tiles each -> 13 splits.
     assert ws(1, 16, 32, 8, 16, 4000) == 13 * 16 * 32 * 128 * 4 + 13 * 16 * 32 * 2 * 4
     assert ws(1, 16, 32, 8, 16, 200) == 0            # too few keys to split
+    # 300 queries x 2 over 5000 keys: 80 workgroups of 79 tiles -> 3 splits of
+    # 27 (one round of 240), not 4 of 20 (320 workgroups, two rounds).
+    assert ws(2, 600, 32, 8, 300, 5000) == 3 * 600 * 32 * 128 * 4 + 3 * 600 * 32 * 2 * 4
+    # 100 queries x 3 over 4100 keys: 48 workgroups of 65 tiles -> 5 splits of 13.
+    assert ws(3, 300, 32, 8, 100, 4100) == 5 * 300 * 32 * 128 * 4 + 5 * 300 * 32 * 2 * 4
     assert ws(8, 8 * 4096, 32, 8, 4096, 8192) == 0   # config-3-sized grid fills the chip
     assert ws(0, 0, 32, 8, 16, 16384) == 0
     assert ws(1, 16, 32, 5, 16, 16384) == 0          # group size not 4 or 8
