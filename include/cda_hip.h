@@ -370,6 +370,24 @@ int cda_fa2_paged_cache_to_dense_rotated_k4v2(const void *kv_cache, int64_t num_
                                               int max_seq_len, void *k_out, void *v_out,
                                               void *stream);
 
+/* The pair cda_fa2_paged_cache_to_dense_rotated + cda_fa2_varlen_fwd_hadamard
+ * that fa2_cda_prefill_varlen_v1 runs (cda/kernels_cuda/fa2_cda.py:98-230) for
+ * callers that do not need the dense K/V: they live in the workspace, sequence
+ * b's rows at b * max_seq_len, and only the rows of seq_lens[b] keys are
+ * written.  Arguments as cda_prefill_paged_hadamard; levels_v 16 (K4V4) or 4
+ * (the K4V2 slot), keys past max_seq_len are not visible.
+ *   workspace: 256-byte aligned device scratch of at least
+ *              cda_prefill_dense_workspace_size(B, H_kv, max_seq_len) bytes.
+ * Calls sharing one workspace must not overlap. */
+size_t cda_prefill_dense_workspace_size(int B, int H_kv, int max_seq_len);
+int cda_prefill_dense_hadamard(const void *q, const void *kv_cache, int64_t num_slots,
+                               int slot_bytes, int H_kv, const int32_t *block_table,
+                               int bt_stride, const int32_t *cu_seqlens_q,
+                               const int32_t *seq_lens, int B, const float *cb_k,
+                               const float *cb_v, int levels_v, void *out, int T, int H_q,
+                               int block_size, int max_query_len, int max_seq_len, float scale,
+                               void *workspace, size_t workspace_bytes, void *stream);
+
 /* Replaces the reference pybind function hadamard128_fp16(x, y, scale)
  * (cda/kernels_cuda/fa2_cda.py:51-52, module _v1_fa2_cda_hadamard128):
  * y = fp16(scale * x @ H_128) for `rows` rows of 128 fp16, H the unnormalised

@@ -40,6 +40,8 @@ SYMBOLS = (
     "cda_prefill_workspace_size",
     "cda_prefill_paged_hadamard_ws",
     "cda_fa2_varlen_fwd_hadamard",
+    "cda_prefill_dense_workspace_size",
+    "cda_prefill_dense_hadamard",
     "cda_fa2_varlen_fwd",
     "cda_fa2_varlen_fwd_lse",
     "cda_dequantize_rows",
@@ -128,6 +130,12 @@ def lib():
         L.cda_prefill_paged_hadamard.argtypes = [
             _P, _P, _I64, _I32, _I32, _P, _I32, _P, _P, _I32, _P, _P, _I32, _P, _I32, _I32,
             _I32, _I32, _F32, _P]
+        L.cda_prefill_dense_workspace_size.restype = _SZ
+        L.cda_prefill_dense_workspace_size.argtypes = [_I32, _I32, _I32]
+        L.cda_prefill_dense_hadamard.restype = _I32
+        L.cda_prefill_dense_hadamard.argtypes = [
+            _P, _P, _I64, _I32, _I32, _P, _I32, _P, _P, _I32, _P, _P, _I32, _P, _I32, _I32,
+            _I32, _I32, _I32, _F32, _P, _SZ, _P]
         L.cda_prefill_workspace_size.restype = _SZ
         L.cda_prefill_workspace_size.argtypes = [_I32, _I32, _I32, _I32, _I32, _I32]
         L.cda_prefill_paged_hadamard_ws.restype = _I32

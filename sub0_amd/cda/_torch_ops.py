@@ -13,7 +13,7 @@ file themselves.
 ``torch.ops.cda_hip`` -- the product entry points the reference reaches
 through its pybind modules (``cda/kernels_cuda/wrappers.py:115-124,
 153-156``, ``fa2_cda.py:51-52, 85-95, 166-181``): ``decode``, ``encode``,
-``decode_uniform_qk``, ``qk_scores_uniform4``, ``prefill``, ``prefill_hybrid``,
+``decode_uniform_qk``, ``qk_scores_uniform4``, ``prefill``, ``prefill_dense``, ``prefill_hybrid``,
 ``paged_to_dense``, ``varlen_fwd_hadamard``, ``varlen_fwd``, ``hadamard128``.
 ``load_pybind_module`` routes its module functions through these ops.
 

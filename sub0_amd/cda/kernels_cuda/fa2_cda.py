@@ -144,7 +144,14 @@ def fa2_cda_prefill_varlen_v1(
     # kernel reads K4V4 slots).
     dense = return_dense_kv or k4v2 or prefill_source(B, kv.shape[-2], int(max_query_len),
                                                       int(max_seq_len)) == "dense"
-    if dense:
+    if dense and not return_dense_kv:
+        load_fa2_cda_loader(k4v2=k4v2)   # same artefact family as the reference's bridge
+        load_fa2_cda_varlen_fused()
+        torch.ops.cda_hip.prefill_dense(
+            Q_in.contiguous(), kv, bt, cu_q.contiguous(), sl.contiguous(), cb_K.contiguous(),
+            cb_V.contiguous(), out, int(block_size), int(max_query_len), int(max_seq_len),
+            float(scale))
+    elif dense:
         k_rot, v_rot = paged_cache_to_dense_rotated(kv, bt, sl, cb_K=cb_K, cb_V=cb_V,
                                                     block_size=block_size,
                                                     max_seq_len=max_seq_len, k4v2=k4v2)

@@ -187,7 +187,8 @@ struct PrefillParams {
     const float *cb_k, *cb_v;
     // dense source
     const uint16_t *k_rot, *v_rot;
-    const int32_t *cu_k;        // (B+1,) first dense row of each sequence
+    const int32_t *cu_k;        // (B+1,) first dense row of each sequence, or null:
+    int dense_stride;           // sequence b's rows are [b * dense_stride, +dense_stride)
     // key split (n_ksplit > 1): split ks of a query block takes key tiles
     // [ks * ksplit_tiles, +ksplit_tiles) and writes unnormalised partials
     // (rotated frame) instead of out; prefill_combine_kernel merges them.
@@ -415,6 +416,7 @@ prefill_kernel(PrefillParams p) {
     const int seq_q = p.cu_q[b + 1] - q_begin;
     const int seq_k = p.key_range == kKeysPast    ? max(0, p.seq_k[b] - seq_q)
                       : p.key_range == kKeysChunk ? seq_q
+                      : (!PAGED && !p.cu_k)       ? min(p.seq_k[b], p.dense_stride)
                                                   : p.seq_k[b];
     // Longest workgroups first: blockIdx.x counts query blocks from the end.
     // Consecutive workgroups share one (sequence, KV head) and so read the
@@ -607,7 +609,7 @@ prefill_kernel(PrefillParams p) {
     // costs speed, never keys.
     const int jt1 = (KSPLIT && ks < p.n_ksplit - 1) ? min(ntiles, jt0 + p.ksplit_tiles) : ntiles;
     const int32_t *bt_row = PAGED ? p.block_table + (int64_t)b * p.bt_stride : nullptr;
-    const int64_t dense_row0 = PAGED ? 0 : p.cu_k[b];
+    const int64_t dense_row0 = PAGED ? 0 : p.cu_k ? p.cu_k[b] : (int64_t)b * p.dense_stride;
     TileRegs cur;
     TileRows rows_next{0, 0};
     // Dense source: K tile j into LDS buffer j & 1 by DMA, two instructions per
@@ -771,29 +773,34 @@ prefill_kernel(PrefillParams p) {
 
 // Dense rotated K/V from the paged cache (fa2_cda.py:64-95): row b*max_seq + t
 // of (B*max_seq, H_kv, 128) fp16 = fp16(centroid * norm) for t < seq_lens[b],
-// zeros beyond.  One 256-thread block per (4 rows of one sequence); thread =
-// (row, head, 16-dim chunk); the per-code tables sit in LDS (64 lane columns).
+// zeros up to max_seq (zero_tail) or, where only the rows of seq_lens[b] keys
+// will be read, up to seq_lens[b]: a quarter to half of the writes of a ragged
+// batch.  One 256-thread block per (kDenseRows rows of one sequence); thread = (row,
+// head, 16-dim chunk); the per-code tables sit in LDS (64 lane columns).
+constexpr int kDenseRows = 4;
 template <int LV>
 __global__ void __launch_bounds__(256)
 paged_to_dense_kernel(const uint8_t *kv, int64_t row_bytes, int slot_bytes, int H_kv,
                       const int32_t *block_table, int bt_stride, const int32_t *seq_lens,
                       const float *cb_k, const float *cb_v, int block_size, int max_seq,
-                      uint16_t *k_out, uint16_t *v_out) {
+                      int zero_tail, uint16_t *k_out, uint16_t *v_out) {
     __shared__ float lut[2][16 * 64];
     const int tid = threadIdx.x;
+    const int b = blockIdx.y;
+    const int rows = zero_tail ? max_seq : min(seq_lens[b], max_seq);
+    if ((int)blockIdx.x * kDenseRows >= rows) return;
     for (int i = tid; i < 2 * 16 * 64; i += 256)
         lut[i >> 10][i & 1023] = (i < 1024) ? cb_k[(i & 1023) >> 6]
                                             : (((i & 1023) >> 6) < LV ? cb_v[(i & 1023) >> 6] : 0.0f);
     __syncthreads();
-    const int b = blockIdx.y;
     const int n = min(seq_lens[b], bt_stride * block_size);
     const uint32_t col = (uint32_t)(tid & 63) * 4u;
     const uint8_t *lk = reinterpret_cast<const uint8_t *>(lut[0]);
     const uint8_t *lv = reinterpret_cast<const uint8_t *>(lut[1]);
     const int per_row = H_kv * 8;                       // threads per token row
-    for (int w = tid; w < 4 * per_row; w += 256) {
-        const int t = blockIdx.x * 4 + w / per_row;
-        if (t >= max_seq) break;
+    for (int w = tid; w < kDenseRows * per_row; w += 256) {
+        const int t = blockIdx.x * kDenseRows + w / per_row;
+        if (t >= rows) break;
         const int h = (w % per_row) >> 3, c = w & 7;    // dims [16c, 16c+16)
         uint4 ko0 = make_uint4(0, 0, 0, 0), ko1 = ko0, vo0 = ko0, vo1 = ko0;
         if (t < n) {
@@ -1163,9 +1170,10 @@ int fa2_varlen_dense(const void *q, const void *k, const void *v, void *out,
                      const int32_t *cu_seqlens_q, const int32_t *cu_seqlens_k,
                      const int32_t *seqused_k, int B, int T, int H_q, int H_kv,
                      int max_query_len, float scale, int causal, int rotate, float *lse,
-                     void *stream, const char *fn) {
+                     void *stream, const char *fn, int dense_stride = 0) {
+    // Keys: cu_seqlens_k, or sequence b's rows at b * dense_stride.
     const std::string f(fn);
-    CDA_REQUIRE(q && k && v && out && cu_seqlens_q && cu_seqlens_k && seqused_k,
+    CDA_REQUIRE(q && k && v && out && cu_seqlens_q && (cu_seqlens_k || dense_stride > 0) && seqused_k,
                 f + ": null pointer argument");
     CDA_REQUIRE(B >= 0 && H_kv > 0 && H_q > 0 && max_query_len >= 0,
                 f + ": bad B / H_q / H_kv / max_query_len");
@@ -1188,6 +1196,7 @@ int fa2_varlen_dense(const void *q, const void *k, const void *v, void *out,
     p.k_rot = static_cast<const uint16_t *>(k);
     p.v_rot = static_cast<const uint16_t *>(v);
     p.cu_k = cu_seqlens_k;
+    p.dense_stride = dense_stride;
     p.n_ksplit = 1;
     p.T_total = T;
     p.rotate = rotate;
@@ -1321,7 +1330,7 @@ namespace {
 int paged_to_dense_impl(const void *kv_cache, int slot_bytes, int H_kv, const int32_t *block_table,
                         int bt_stride, const int32_t *seq_lens, int B, const float *cb_k,
                         const float *cb_v, int levels_v, int block_size, int max_seq_len,
-                        void *k_out, void *v_out, void *stream, const char *fn) {
+                        void *k_out, void *v_out, int zero_tail, void *stream, const char *fn) {
     const std::string f(fn);
     CDA_REQUIRE(kv_cache && block_table && seq_lens && cb_k && cb_v && k_out && v_out,
                 f + ": null pointer argument");
@@ -1335,7 +1344,7 @@ int paged_to_dense_impl(const void *kv_cache, int slot_bytes, int H_kv, const in
                     ((uintptr_t)v_out & 15) == 0,
                 f + ": misaligned pointer");
     if (B == 0 || max_seq_len == 0) return CDA_OK;
-    const dim3 grid((max_seq_len + 3) / 4, B);
+    const dim3 grid((max_seq_len + kDenseRows - 1) / kDenseRows, B);
     hipStream_t st = static_cast<hipStream_t>(stream);
     const auto *kv = static_cast<const uint8_t *>(kv_cache);
     const int64_t row = (int64_t)H_kv * slot_bytes;
@@ -1344,11 +1353,11 @@ int paged_to_dense_impl(const void *kv_cache, int slot_bytes, int H_kv, const in
     if (levels_v == 16)
         paged_to_dense_kernel<16><<<grid, 256, 0, st>>>(kv, row, slot_bytes, H_kv, block_table,
                                                         bt_stride, seq_lens, cb_k, cb_v,
-                                                        block_size, max_seq_len, ko, vo);
+                                                        block_size, max_seq_len, zero_tail, ko, vo);
     else
         paged_to_dense_kernel<4><<<grid, 256, 0, st>>>(kv, row, slot_bytes, H_kv, block_table,
                                                        bt_stride, seq_lens, cb_k, cb_v,
-                                                       block_size, max_seq_len, ko, vo);
+                                                       block_size, max_seq_len, zero_tail, ko, vo);
     CDA_LAUNCH_CHECK(f + ": paged_to_dense_kernel");
     return CDA_OK;
 }
@@ -1365,7 +1374,7 @@ extern "C" int cda_fa2_paged_cache_to_dense_rotated(const void *kv_cache, int64_
     (void)num_slots;
     CDA_REQUIRE(levels == 16, "cda_fa2_paged_cache_to_dense_rotated: K4V4 caches only (16 levels)");
     return paged_to_dense_impl(kv_cache, slot_bytes, H_kv, block_table, bt_stride, seq_lens, B,
-                               cb_k, cb_v, 16, block_size, max_seq_len, k_out, v_out, stream,
+                               cb_k, cb_v, 16, block_size, max_seq_len, k_out, v_out, 1, stream,
                                "cda_fa2_paged_cache_to_dense_rotated");
 }
 
@@ -1375,8 +1384,41 @@ extern "C" int cda_fa2_paged_cache_to_dense_rotated_k4v2(
     int block_size, int max_seq_len, void *k_out, void *v_out, void *stream) {
     (void)num_slots;
     return paged_to_dense_impl(kv_cache, slot_bytes, H_kv, block_table, bt_stride, seq_lens, B,
-                               cb_k, cb_v, 4, block_size, max_seq_len, k_out, v_out, stream,
+                               cb_k, cb_v, 4, block_size, max_seq_len, k_out, v_out, 1, stream,
                                "cda_fa2_paged_cache_to_dense_rotated_k4v2");
+}
+
+extern "C" size_t cda_prefill_dense_workspace_size(int B, int H_kv, int max_seq_len) {
+    if (B <= 0 || H_kv <= 0 || max_seq_len <= 0) return 0;
+    return 2 * align256((size_t)B * max_seq_len * H_kv * cda::kD * 2);
+}
+
+extern "C" int cda_prefill_dense_hadamard(const void *q, const void *kv_cache, int64_t num_slots,
+                                          int slot_bytes, int H_kv, const int32_t *block_table,
+                                          int bt_stride, const int32_t *cu_seqlens_q,
+                                          const int32_t *seq_lens, int B, const float *cb_k,
+                                          const float *cb_v, int levels_v, void *out, int T,
+                                          int H_q, int block_size, int max_query_len,
+                                          int max_seq_len, float scale, void *workspace,
+                                          size_t workspace_bytes, void *stream) {
+    const char *fn = "cda_prefill_dense_hadamard";
+    (void)num_slots;
+    CDA_REQUIRE(levels_v == 16 || levels_v == 4,
+                "cda_prefill_dense_hadamard: K4V4 or K4V2 caches (V codebook of 16 or 4 levels)");
+    CDA_REQUIRE(max_seq_len > 0 || B == 0 || max_query_len == 0,
+                "cda_prefill_dense_hadamard: max_seq_len must be > 0");
+    if (B == 0 || max_query_len == 0) return CDA_OK;
+    const size_t need = cda_prefill_dense_workspace_size(B, H_kv, max_seq_len);
+    if (!workspace || workspace_bytes < need || need == 0 || ((uintptr_t)workspace & 255))
+        return fail(CDA_E_WORKSPACE, "cda_prefill_dense_hadamard: workspace missing, misaligned "
+                                     "or smaller than cda_prefill_dense_workspace_size()");
+    void *k_rot = workspace, *v_rot = static_cast<char *>(workspace) + need / 2;
+    const int rc = paged_to_dense_impl(kv_cache, slot_bytes, H_kv, block_table, bt_stride, seq_lens,
+                                       B, cb_k, cb_v, levels_v, block_size, max_seq_len, k_rot,
+                                       v_rot, 0, stream, fn);
+    if (rc != CDA_OK) return rc;
+    return fa2_varlen_dense(q, k_rot, v_rot, out, cu_seqlens_q, nullptr, seq_lens, B, T, H_q, H_kv,
+                            max_query_len, scale, 1, 1, nullptr, stream, fn, max_seq_len);
 }
 
 extern "C" int cda_hadamard128_fp16(const void *x, void *y, int64_t rows, float scale,

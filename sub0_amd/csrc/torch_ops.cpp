@@ -302,6 +302,35 @@ void prefill(const Tensor &q, const Tensor &kv, const Tensor &bt, const Tensor &
              "cda_prefill_paged_hadamard_ws");
 }
 
+// Prefill through dense K/V held in scratch (the bridge without its results).
+void prefill_dense(const Tensor &q, const Tensor &kv, const Tensor &bt, const Tensor &cu_q,
+                   const Tensor &sl, const Tensor &cb_k, const Tensor &cb_v, const Tensor &out,
+                   int64_t bs, int64_t max_query_len, int64_t max_seq_len, double scale) {
+    const DeviceGuard guard(on_gpu({&q, &kv, &bt, &cu_q, &sl, &cb_k, &cb_v, &out}));
+    check_paged(kv, bt, sl, cb_k, cb_v, true);
+    TORCH_CHECK_TYPE(q.scalar_type() == at::kHalf && out.scalar_type() == at::kHalf,
+                     "Q and output must be fp16");
+    TORCH_CHECK_VALUE(q.dim() == 3 && q.size(2) == 128 && q.is_contiguous(),
+                      "Q must be a contiguous (rows, heads, 128) tensor");
+    TORCH_CHECK_VALUE(out.sizes() == q.sizes() && out.is_contiguous(),
+                      "output must be a contiguous tensor shaped like Q");
+    need_dtype(cu_q, at::kInt, "cu_seqlens_q must be int32");
+    const int B = (int)cu_q.numel() - 1;
+    TORCH_CHECK_VALUE(sl.numel() >= B && bt.size(0) >= B,
+                      "seq_lens / block_table have fewer rows than cu_seqlens_q");
+    const int H_kv = (int)kv.size(1);
+    const Tensor ck = f32c(cb_k), cv = f32c(cb_v);
+    Workspace ws = workspace(q, cda_prefill_dense_workspace_size(B, H_kv, (int)max_seq_len));
+    check_rc(cda_prefill_dense_hadamard(
+                 q.data_ptr(), kv.data_ptr(), kv.size(0), (int)kv.size(2), H_kv,
+                 bt.data_ptr<int32_t>(), (int)bt.stride(0), cu_q.data_ptr<int32_t>(),
+                 sl.data_ptr<int32_t>(), B, ck.data_ptr<float>(), cv.data_ptr<float>(),
+                 (int)cv.numel(), out.data_ptr(), (int)q.size(0), (int)q.size(1), (int)bs,
+                 (int)max_query_len, (int)max_seq_len, (float)scale, ws.ptr, ws.bytes,
+                 stream_of(q)),
+             "cda_prefill_dense_hadamard");
+}
+
 void prefill_hybrid(const Tensor &q, const Tensor &k_new, const Tensor &v_new, const Tensor &kv,
                     const Tensor &bt, const Tensor &cu_q, const Tensor &sl, const Tensor &cb_k,
                     const Tensor &cb_v, const Tensor &out, int64_t bs, int64_t max_query_len,
@@ -588,6 +617,9 @@ void nothing_scores(const Tensor &, const Tensor &, const Tensor &, const Tensor
                     double, bool, int64_t, int64_t, int64_t) {}
 void nothing_encode(const Tensor &, const Tensor &, const Tensor &, const Tensor &,
                     const Tensor &, const Tensor &) {}
+void nothing_prefill_dense(const Tensor &, const Tensor &, const Tensor &, const Tensor &,
+                           const Tensor &, const Tensor &, const Tensor &, const Tensor &, int64_t,
+                           int64_t, int64_t, double) {}
 void nothing_prefill(const Tensor &, const Tensor &, const Tensor &, const Tensor &,
                      const Tensor &, const Tensor &, const Tensor &, const Tensor &, int64_t,
                      int64_t, double, int64_t) {}
@@ -667,6 +699,9 @@ TORCH_LIBRARY(cda_hip, m) {
           "int key_end) -> ()");
     m.def("encode(Tensor k, Tensor v, Tensor slot_mapping, Tensor(a!) flat_cache, Tensor cb_k, "
           "Tensor cb_v) -> ()");
+    m.def("prefill_dense(Tensor q, Tensor kv_cache, Tensor block_table, Tensor cu_seqlens_q, "
+          "Tensor seq_lens, Tensor cb_k, Tensor cb_v, Tensor(a!) out, int block_size, "
+          "int max_query_len, int max_seq_len, float scale) -> ()");
     m.def("prefill(Tensor q, Tensor kv_cache, Tensor block_table, Tensor cu_seqlens_q, "
           "Tensor seq_lens, Tensor cb_k, Tensor cb_v, Tensor(a!) out, int block_size, "
           "int max_query_len, float scale, int max_seq_len=-1) -> ()");
@@ -690,6 +725,7 @@ TORCH_LIBRARY_IMPL(cda_hip, CUDA, m) {
     m.impl("qk_scores_uniform4", &qk_scores_uniform4);
     m.impl("encode", &encode);
     m.impl("prefill", &prefill);
+    m.impl("prefill_dense", &prefill_dense);
     m.impl("prefill_hybrid", &prefill_hybrid);
     m.impl("varlen_fwd", &varlen_fwd);
     m.impl("paged_to_dense", &paged_to_dense);
@@ -703,6 +739,7 @@ TORCH_LIBRARY_IMPL(cda_hip, Meta, m) {
     m.impl("qk_scores_uniform4", &nothing_scores);
     m.impl("encode", &nothing_encode);
     m.impl("prefill", &nothing_prefill);
+    m.impl("prefill_dense", &nothing_prefill_dense);
     m.impl("prefill_hybrid", &nothing_hybrid);
     m.impl("varlen_fwd", &nothing_varlen);
     m.impl("paged_to_dense", &meta_paged_to_dense);

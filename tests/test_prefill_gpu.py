@@ -273,3 +273,29 @@ def test_prefill_key_split_padded_query_rows(gpu):
     out = run_prefill(case, gpu, split=True, pad_rows=5)
     check(out[:12], case.expected)
     assert np.isnan(out[12:]).all()
+
+
+@pytest.mark.parametrize("seq_q,seq_k,H_kv,gs,slack", [
+    ([300, 1, 77], [300, 1000, 77], 8, 4, 0),
+    ([64], [65], 2, 8, 63),
+    ([5, 513, 0], [5, 513, 40], 1, 4, 1),
+])
+def test_prefill_dense_scratch_matches_bridge(gpu, seq_q, seq_k, H_kv, gs, slack):
+    """The dense prefill with its K/V in scratch (rows past a sequence's keys
+    are not written) gives the bits of the two-call bridge, and the checker's
+    output within the tolerance; the scratch starts as NaN."""
+    print(f"[prefill-dense] seq_q={seq_q} seq_k={seq_k} H_kv={H_kv}", flush=True)
+    case = make_prefill_case(6100 + slack, seq_q, seq_k, H_kv=H_kv, gs=gs, fill=0xFF)
+    bridge = run_prefill(case, gpu, dense=True)
+    q, cache, bt = (_dev(x, gpu) for x in (case.q, case.cache, case.block_table))
+    cu, sk, cb = (_dev(x, gpu) for x in (case.cu_q, case.seq_k, case.cb))
+    # What the caching allocator hands the op next: the pattern of a NaN.
+    junk = torch.full((1 << 24,), 0xFF, dtype=torch.uint8, device=gpu)
+    del junk
+    out = torch.full_like(q, float("nan"))
+    torch.ops.cda_hip.prefill_dense(q, cache, bt, cu, sk, cb, cb, out, case.block_size,
+                                    max(seq_q), max(seq_k) + slack, float(1 / np.sqrt(128)))
+    torch.cuda.synchronize()
+    out = out.cpu().numpy()
+    assert np.array_equal(out.view(np.uint16), bridge.view(np.uint16))
+    check(out, case.expected)
