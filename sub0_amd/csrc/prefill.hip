@@ -74,6 +74,12 @@ constexpr int kPrefillLds = kLutOff + kLutBytes;
 // chunk p ^ (k & 15), and the 16 lanes of an MFMA operand read (rows c32,
 // chunk 2S + u) then fall in 16 distinct bank groups.
 constexpr int kKRowDense = kD * 2;                      // 256
+// The V tile of the dense source is copied the same way, row-major, chunk c of
+// key k at position c ^ 4 * (k & 3), and transposed by the operand reads
+// (ds_read_b64_tr_b16: each 16 lanes read four rows of 16 columns, lane i gets
+// column i): with that order the 8 rows x 64 bytes of one read fall on all 64
+// banks twice.  Passing V through registers into a V^T tile (loads, a 4 x 4
+// transpose, four stores a thread, all between two barriers) took @@.
 
 typedef unsigned v4u32 __attribute__((ext_vector_type(4)));
 
@@ -86,6 +92,15 @@ __device__ __forceinline__ void dma_x4_to_lds(v4u32 rsrc, uint32_t voff, uint32_
     asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\t"
                  "buffer_load_dwordx4 %1, %2, 0 offen lds\n\ts_mov_b32 m0, %0"
                  : "=&s"(saved) : "v"(voff), "s"(rsrc), "s"(lds_base) : "memory");
+}
+
+// Four keys' values of this lane's dim from a row-major tile: lane i of 16
+// passes the address of row i >> 2, columns 4 * (i & 3) .. + 3, and receives
+// column i of the four rows.
+typedef short short4v __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ uint2 lds_read_tr(uint32_t addr) {
+    return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                         (__attribute__((address_space(3))) short4v *)addr));
 }
 
 __device__ __forceinline__ uint32_t lds_addr32(const void *ptr) {
@@ -216,12 +231,11 @@ struct PrefillParams {
 };
 constexpr int kKeysAll = 0, kKeysPast = 1, kKeysChunk = 2;
 
-// Registers holding one tile's share of the source data for this thread:
-// paged: K codes k[0..1] + nk, V codes v[0..3] (two bytes per key) + nv[];
-// dense: K fp16 k[0..7], V fp16 v[2i], v[2i+1] for key i.
+// Registers holding one tile's share of the paged source for this thread:
+// K codes k[0..1] + nk, V codes v[0..3] (two bytes per key) + nv[].
 struct TileRegs {
-    uint32_t k[8];
-    uint32_t v[8];
+    uint32_t k[2];
+    uint32_t v[4];
     float nk;
     float nv[4];
 };
@@ -253,12 +267,10 @@ __device__ __forceinline__ TileRows fetch_rows(const PrefillParams &p, const int
 // Source loads of one tile.  K share: key tk = tid >> 3, dims [16c, 16c+16)
 // with c = tid & 7.  V share: keys 4g..4g+3 with g = v_gv(tid), dims
 // [4c, 4c+4) with c = v_cv(tid).  Keys at or past nk_valid are not read
-// (zeros; they are masked later).  Dense rows start at dense_row0 (the
-// sequence's first row of k_rot / v_rot).
+// (zeros; they are masked later).  The dense source goes by DMA instead.
 template <bool PAGED>
 __device__ __forceinline__ void load_tile(const PrefillParams &p, TileRegs &r, TileRows rows,
-                                          int64_t dense_row0, int h, int kbase, int nk_valid,
-                                          int tid) {
+                                          int h, int kbase, int nk_valid, int tid) {
     const int tk = tid >> 3, ck = tid & 7;
     const int gv = v_gv(tid), cv = v_cv(tid);
     if (PAGED) {
@@ -289,21 +301,6 @@ __device__ __forceinline__ void load_tile(const PrefillParams &p, TileRegs &r, T
                 r.nv[i] = *reinterpret_cast<const float *>(rp + 132);
             }
         }
-    } else {
-        // Dense rows and the row pitch are below 2^31: 32 x 32 -> 64-bit multiplies.
-        // The K tile goes by DMA (issue_k_dma); only V passes through registers.
-        (void)tk;
-        (void)ck;
-        const uint32_t r0 = (uint32_t)(dense_row0 + kbase);
-        const uint32_t hs = (uint32_t)(p.H_kv * kD);
-        const uint16_t *vrow = p.v_rot + (uint64_t)(r0 + 4 * gv) * hs + h * kD + 4 * cv;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            uint2 v = make_uint2(0u, 0u);
-            if (4 * gv + i < nk_valid) v = *reinterpret_cast<const uint2 *>(vrow + (size_t)i * hs);
-            r.v[2 * i] = v.x;
-            r.v[2 * i + 1] = v.y;
-        }
     }
 }
 
@@ -332,32 +329,21 @@ __device__ __forceinline__ uint32_t dq_pair(const uint8_t *lut, uint32_t byte, u
     return cvt_pk(hi * norm, lo * norm);
 }
 
-template <bool PAGED>
 __device__ __forceinline__ void store_tile(const TileRegs &r, uint8_t *kt, uint8_t *vt,
                                            const uint8_t *lutk, const uint8_t *lutv, int tid) {
     const int tk = tid >> 3, ck = tid & 7;
     const int gv = v_gv(tid), cv = v_cv(tid);
     uint32_t kw[8];      // key tk, dims [16ck, 16ck+16) as fp16 pairs (2j, 2j+1)
     uint32_t pr[4][2];   // key 4gv+i: dims (4cv, 4cv+1), (4cv+2, 4cv+3) as fp16 pairs
-    if (PAGED) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const uint32_t byte = (r.k[j >> 2] >> (8 * (j & 3))) & 0xFFu;
-            kw[j] = dq_byte(lutk, byte, r.nk);
-        }
+    for (int j = 0; j < 8; ++j) {
+        const uint32_t byte = (r.k[j >> 2] >> (8 * (j & 3))) & 0xFFu;
+        kw[j] = dq_byte(lutk, byte, r.nk);
+    }
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            pr[i][0] = dq_byte(lutv, r.v[i] & 0xFFu, r.nv[i]);
-            pr[i][1] = dq_byte(lutv, (r.v[i] >> 8) & 0xFFu, r.nv[i]);
-        }
-    } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) kw[j] = 0u;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            pr[i][0] = r.v[2 * i];
-            pr[i][1] = r.v[2 * i + 1];
-        }
+    for (int i = 0; i < 4; ++i) {
+        pr[i][0] = dq_byte(lutv, r.v[i] & 0xFFu, r.nv[i]);
+        pr[i][1] = dq_byte(lutv, (r.v[i] >> 8) & 0xFFu, r.nv[i]);
     }
     // V^T: dim 4cv+k gets keys 4gv..4gv+3 (a 4 x 4 fp16 transpose).
     uint32_t vw[4][2];
@@ -368,11 +354,9 @@ __device__ __forceinline__ void store_tile(const TileRegs &r, uint8_t *kt, uint8
         vw[k][0] = __builtin_amdgcn_perm(pr[1][w], pr[0][w], sel);
         vw[k][1] = __builtin_amdgcn_perm(pr[3][w], pr[2][w], sel);
     }
-    if (PAGED) {
-        uint4 *kd = reinterpret_cast<uint4 *>(kt + tk * kKRow + 32 * ck);
-        kd[0] = make_uint4(kw[0], kw[1], kw[2], kw[3]);
-        kd[1] = make_uint4(kw[4], kw[5], kw[6], kw[7]);
-    }
+    uint4 *kd = reinterpret_cast<uint4 *>(kt + tk * kKRow + 32 * ck);
+    kd[0] = make_uint4(kw[0], kw[1], kw[2], kw[3]);
+    kd[1] = make_uint4(kw[4], kw[5], kw[6], kw[7]);
     const uint32_t vo = v_key_off(gv);
 #pragma unroll
     for (int k = 0; k < 4; ++k)
@@ -490,6 +474,16 @@ prefill_kernel(PrefillParams p) {
         k_off[S] = PAGED ? k_lane + 32u * S
                          : (uint32_t)(c32 * kKRowDense + 16 * ((2 * S + u) ^ (c32 & 15)));
 
+    // Dense source: this lane's V reads of dims 32T .. (key group 0): row 4u + (i
+    // >> 2), i = lane & 15, dims 32T + 16 * (bit 4 of the lane) + 4 * (i & 3).
+    uint32_t v_off[4];
+#pragma unroll
+    for (int T = 0; T < 4; ++T) {
+        const int i = lane & 15, row = 4 * u + (i >> 2);
+        const int chunk = 4 * T + 2 * ((lane >> 4) & 1) + ((i & 3) >> 1);
+        v_off[T] = (uint32_t)(kKTile + row * kKRowDense + 16 * (chunk ^ (4 * (i >> 2))) + 8 * (i & 1));
+    }
+
     // Per 64-key tile: S^T = K q_rot^T; online softmax in the log2 domain with
     // a lazy rescale (the running max moves only when a tile's max exceeds it
     // by more than 8, so P <= 2^8 and the O rescale is rare after the first
@@ -594,8 +588,16 @@ prefill_kernel(PrefillParams p) {
         for (int ks = 0; ks < 4; ++ks) {
             half8 a[4];
 #pragma unroll
-            for (int T = 0; T < 4; ++T)
-                a[T] = *reinterpret_cast<const half8 *>(buf + v_lane + T * 32 * kVRow + 32 * ks);
+            for (int T = 0; T < 4; ++T) {
+                if constexpr (PAGED) {
+                    a[T] = *reinterpret_cast<const half8 *>(buf + v_lane + T * 32 * kVRow + 32 * ks);
+                } else {
+                    // Keys 16ks + 4u .. + 3, then 8 further on: the k order of P^T.
+                    const uint32_t at = lds_addr32(buf) + v_off[T] + ks * 16 * kKRowDense;
+                    const uint2 k0 = lds_read_tr(at), k1 = lds_read_tr(at + 8 * kKRowDense);
+                    a[T] = __builtin_bit_cast(half8, make_uint4(k0.x, k0.y, k1.x, k1.y));
+                }
+            }
             const half8 pb = pbs[ks];
 #pragma unroll
             for (int T = 0; T < 4; ++T) o[T] = mfma32(a[T], pb, o[T]);
@@ -612,56 +614,67 @@ prefill_kernel(PrefillParams p) {
     const int64_t dense_row0 = PAGED ? 0 : p.cu_k ? p.cu_k[b] : (int64_t)b * p.dense_stride;
     TileRegs cur;
     TileRows rows_next{0, 0};
-    // Dense source: K tile j into LDS buffer j & 1 by DMA, two instructions per
-    // wave (keys 8*wave .. +7).  Keys past the end of the tile's valid range
-    // read the last valid key's row (in bounds; their scores are masked).
-    auto issue_k_dma = [&](int j) CDA_INLINE {
+    // Dense source: tile j into LDS buffer j & 1 by DMA, two instructions per
+    // wave for K and two for V (keys 8*wave .. +7).  Keys past the end of the
+    // tile's valid range read the last valid key's row (in bounds; their
+    // scores are masked and their weights 0).
+    auto issue_dma = [&](int j) CDA_INLINE {
         if constexpr (!PAGED) {
             const int kb = j * kBN;
             const int nk_valid = min(kBN, kend - kb);
             const uint32_t pitch = (uint32_t)(p.H_kv * kD * 2);
-            const uint64_t base =
-                (uint64_t)(p.k_rot + ((uint64_t)(dense_row0 + kb) * p.H_kv + h) * kD);
-            const v4u32 r = {(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)base),
+            const uint64_t row0 = ((uint64_t)(dense_row0 + kb) * p.H_kv + h) * kD;
+            auto rsrc = [&](const uint16_t *rows) CDA_INLINE {
+                const uint64_t base = (uint64_t)(rows + row0);
+                return v4u32{(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)base),
                              (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(base >> 32)) & 0xFFFFu,
                              (uint32_t)(kBN * pitch), 0x00020000u};
+            };
+            const v4u32 rk = rsrc(p.k_rot), rv = rsrc(p.v_rot);
             const uint32_t dst = __builtin_amdgcn_readfirstlane(lds_addr32(smem)) +
                                  (uint32_t)((j & 1) * kTileBytes);
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
                 const int ins = 2 * wave + t;               // keys 4*ins .. 4*ins + 3
                 const int key = 4 * ins + (lane >> 4);
-                const int pos = lane & 15;
-                const uint32_t voff =
-                    (uint32_t)min(key, nk_valid - 1) * pitch + 16u * (uint32_t)(pos ^ (key & 15));
-                dma_x4_to_lds(r, voff, dst + 1024u * (uint32_t)ins);
+                const uint32_t pos = lane & 15, row = (uint32_t)min(key, nk_valid - 1) * pitch;
+                dma_x4_to_lds(rk, row + 16u * (pos ^ (uint32_t)(key & 15)), dst + 1024u * (uint32_t)ins);
+                dma_x4_to_lds(rv, row + 16u * (pos ^ (uint32_t)(4 * (lane >> 4))),
+                              dst + kKTile + 1024u * (uint32_t)ins);
             }
         }
     };
     if (jt0 < jt1) {
         const int k0 = jt0 * kBN, k1 = k0 + kBN;
-        issue_k_dma(jt0);
-        load_tile<PAGED>(p, cur, fetch_rows<PAGED>(p, bt_row, k0, min(kBN, kend - k0), tid),
-                         dense_row0, h, k0, min(kBN, kend - k0), tid);
-        if (jt0 + 1 < jt1) rows_next = fetch_rows<PAGED>(p, bt_row, k1, min(kBN, kend - k1), tid);
+        issue_dma(jt0);
+        if constexpr (PAGED) {
+            load_tile<PAGED>(p, cur, fetch_rows<PAGED>(p, bt_row, k0, min(kBN, kend - k0), tid), h,
+                             k0, min(kBN, kend - k0), tid);
+            if (jt0 + 1 < jt1)
+                rows_next = fetch_rows<PAGED>(p, bt_row, k1, min(kBN, kend - k1), tid);
+        }
     }
     __syncthreads();   // tables visible
 
-    // Tile j into LDS (the whole workgroup), then the loads of tile j + 1.
-    // Dense source: the K DMA of tile j (issued after the previous barrier)
-    // and tile j's V loads are waited for here; the K DMA of tile j + 1 goes
-    // out after this barrier, when every wave is done with buffer (j + 1) & 1.
+    // Tile j ready in LDS for the whole workgroup.  Paged source: the workgroup
+    // stores it, then loads tile j + 1.  Dense source: its DMAs (issued after
+    // the previous barrier) are waited for; those of tile j + 1 go out after
+    // this barrier, when every wave is done with buffer (j + 1) & 1.
     auto produce = [&](int j) CDA_INLINE {
         uint8_t *buf = smem + (j & 1) * kTileBytes;
-        if constexpr (!PAGED) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        store_tile<PAGED>(cur, buf, buf + kKTile, lutk, lutv, tid);
-        if (j + 1 < jt1) {
-            const int k1 = (j + 1) * kBN, k2 = (j + 2) * kBN;
-            load_tile<PAGED>(p, cur, rows_next, dense_row0, h, k1, min(kBN, kend - k1), tid);
-            if (j + 2 < jt1) rows_next = fetch_rows<PAGED>(p, bt_row, k2, min(kBN, kend - k2), tid);
+        if constexpr (PAGED) {
+            store_tile(cur, buf, buf + kKTile, lutk, lutv, tid);
+            if (j + 1 < jt1) {
+                const int k1 = (j + 1) * kBN, k2 = (j + 2) * kBN;
+                load_tile<PAGED>(p, cur, rows_next, h, k1, min(kBN, kend - k1), tid);
+                if (j + 2 < jt1)
+                    rows_next = fetch_rows<PAGED>(p, bt_row, k2, min(kBN, kend - k2), tid);
+            }
+        } else {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         }
         __syncthreads();
-        if (j + 1 < jt1) issue_k_dma(j + 1);
+        if (j + 1 < jt1) issue_dma(j + 1);
         return buf;
     };
     // The tiles whole for every row of this wave come first, those crossing
