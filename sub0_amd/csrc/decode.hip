@@ -1099,17 +1099,22 @@ decode_stream_kernel(SplitParams p) {
                 refill(k);
             }
         } else {
-            // All 64 table reads of the chunk's K codes first, fenced from the
+            // The table reads of two pages' K codes first, fenced from the
             // scheduler, so their LDS latency overlaps instead of stalling
-            // each page's multiplies (534 -> 525 us at B=32, N=64K).
-            float2 cvk[4][16];
+            // each page's multiplies.  All four pages' at once held 64 more
+            // registers and measured no faster (518-520 against 515 us at
+            // B=32, N=64K), one page's 0.1 us slower at B=1, N=4K.
 #pragma unroll
-            for (int k = 0; k < 4; ++k) k_lookup(r[k], cvk[k]);
-            __builtin_amdgcn_sched_barrier(0);
+            for (int k0 = 0; k0 < 4; k0 += 2) {
+                float2 cvk[2][16];
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                sc[k] = k_math(r[k], cvk[k]);
-                refill(k);
+                for (int k = 0; k < 2; ++k) k_lookup(r[k0 + k], cvk[k]);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    sc[k0 + k] = k_math(r[k0 + k], cvk[k]);
+                    refill(k0 + k);
+                }
             }
         }
         float raw[4][4];
@@ -1209,6 +1214,20 @@ decode_stream_kernel(SplitParams p) {
     const int nchunks = (wnpages + 3) >> 2;
     const int nfull = (wend - wstart) >> 6;
     for (int c = 0; c < nfull; ++c) {
+        // The two waves of a SIMD (w, w + 4) take turns at the higher issue
+        // priority, chunk by chunk.  Between equal priorities the older wave
+        // wins, so the younger fell a third behind (loop times 409 and 547 us
+        // at B=32, N=64K) and ended alone on its SIMD, where one wave cannot
+        // fill the issue slots: 2 KV heads x 8 queries, 16 x 4K-16K tokens
+        // 27.0 -> 25.9 us, 512-byte slots 8 x 8K 31.4 -> 30.9, K2V2 32 x 16K
+        // 116.5 -> 114.3, B=32, N=64K 519 -> 507.5 (with the table reads in batches of two pages, above).
+        // (The score-domain form bounds its waves' drift with barriers instead.)
+        if constexpr (!SQK) {
+            if ((c ^ (wave >> 2)) & 1)
+                __builtin_amdgcn_s_setprio(1);
+            else
+                __builtin_amdgcn_s_setprio(0);
+        }
         step(c, std::false_type{});
         if constexpr (SQK) {
             if (c % kSqkSyncChunks == kSqkSyncChunks - 1) __syncthreads();
