@@ -33,6 +33,7 @@
 //                 and writes fp16 out.
 #include "cda_common.h"
 
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 #include <string>
@@ -93,6 +94,11 @@ struct SplitParams {
     uint16_t *out;              // (B, H_q, 128) fp16
     int wave_tokens;            // multiple of 64
     int bs_shift;               // log2(block_size) when it is a power of two, else -1
+    // SLOTS form: the B * n_splits slots are dealt to the sequences by their
+    // lengths, and slots[b] = (first slot, count) is written for the combine.
+    int2 *slots;
+    int B;
+    int max_len;                // tokens of a sequence that are covered
     int xcd_map;                // 1: the heads of a (sequence, split) share an XCD
 };
 
@@ -587,14 +593,15 @@ __device__ __forceinline__ uint32_t bfi(uint32_t m, uint32_t a, uint32_t b) {
 // offset of 128.  With half the columns two lanes of a read share each bank:
 // 4.0 instead of 2.9 cycles per ds_read_b64 and CU, 8.2 instead of 4.1 per
 // ds_read_b128 (2-bit codes), which is why one codebook keeps the full row.
-template <int GS, int L, bool SQK = false, bool FUSED = false, bool TWO = false>
+template <int GS, int L, bool SQK = false, bool FUSED = false, bool TWO = false,
+          bool SLOTS = false>
 __global__ void __launch_bounds__(kThreads, 1)
 decode_stream_kernel(SplitParams p) {
     if (!FUSED && !SQK && p.cb_same && !*p.cb_same) return;   // different codebooks: the general kernel runs
     static_assert(L == 16 || L == 4, "4-bit or 2-bit codes");
     static_assert(!SQK || L == 16, "score-domain QK: 4-bit K codes");
     static_assert(!(SQK && FUSED), "the score-domain form runs as three launches");
-    static_assert(FUSED || !TWO, "two codebooks: single-launch form");
+    static_assert(FUSED || (!TWO && !SLOTS), "two codebooks, slots: single-launch form");
     static_assert(GS == 4 || GS == 8, "GQA groups of 4 or 8");
     // The MFMA's 16 score columns hold the GS heads RP times over, so every
     // lane holds every score of its head RP times.  Each lane computes the
@@ -615,13 +622,14 @@ decode_stream_kernel(SplitParams p) {
     const int r16 = lane & 15;
     const int q4 = lane >> 4;
     int sp, b, h;
+    int tile_n = p.tile_n, n_splits = p.n_splits, wave_tokens = p.wave_tokens;
+    int u = 0;                     // FUSED: slot of this workgroup
     if constexpr (FUSED) {
-        // Linear id -> (unit = (sequence, split), head).  The hardware deals
+        // Linear id -> (slot = (sequence, split), head).  The hardware deals
         // workgroups to the 8 XCDs round-robin by linear id; with xcd_map the
-        // heads of a unit go to one XCD, so the cache lines that neighbouring
+        // heads of a slot go to one XCD, so the cache lines that neighbouring
         // heads' slots share are fetched into one L2.
         const int pl = blockIdx.x;
-        int u;
         if (p.xcd_map) {
             const int i = pl >> 3;
             h = i % p.H_kv;
@@ -637,9 +645,13 @@ decode_stream_kernel(SplitParams p) {
         b = blockIdx.z;
         h = wave;
     }
+    // Lane l: tokens of sequence l (SLOTS).
+    int len_l = 0;
+    if (SLOTS && lane < p.B)
+        len_l = min(min(p.seq_lens[lane], p.bt_stride * p.block_size), p.max_len);
 
     const int bs = p.block_size;
-    const int start = sp * p.tile_n;
+    int start = sp * tile_n;
     // Cache block of token t (FUSED: a shift for the usual block sizes).
     auto block_of = [&](int t) CDA_INLINE {
         return FUSED && p.bs_shift >= 0 ? t >> p.bs_shift : t / bs;
@@ -653,27 +665,74 @@ decode_stream_kernel(SplitParams p) {
     int first_row = 0;
     float cb_lane = 0.0f, rcol[FUSED ? kD / 4 : 1];
     uint16_t qv[FUSED ? kQPer : 1];
-    if constexpr (FUSED) {
+    auto load_own = [&]() CDA_INLINE {
         const int32_t *bt = p.block_table + (int64_t)b * p.bt_stride;
-        const int t0 = start + wave * p.wave_tokens + 16 * (lane & 3);
+        const int t0 = start + wave * wave_tokens + 16 * (lane & 3);
         const int blk = block_of(t0);
         first_row = bt[min(blk, p.bt_stride - 1)] * bs + (t0 - blk * bs);
 #pragma unroll
         for (int i = 0; i < kQPer; ++i)
             qv[i] = p.q[((int64_t)b * p.H_q + (int64_t)h * GS) * kD + tid + i * kThreads];
+    };
+    if constexpr (FUSED) {
+        load_own();
 #pragma unroll
         for (int m = 0; m < kD / 4; ++m)
             rcol[m] = p.R[(4 * m + q4) * kD + 16 * wave + r16];
     }
     if (lane < L) cb_lane = SQK ? p.cb_v[lane] : p.cb_k[lane];
     if (TWO && lane >= 16 && lane < 16 + L) cb_lane = p.cb_v[lane - 16];
-    const int seq_len =
-        __builtin_amdgcn_readfirstlane(min(p.seq_lens[b], p.bt_stride * p.block_size));
-    const int end = min(start + p.tile_n, seq_len);
-    const int64_t part_row = ((int64_t)b * p.n_splits + sp) * p.H_q + (int64_t)h * GS;
+    int seq_len;
+    if constexpr (SLOTS) {
+        // Sequences of one length keep the even split, for which the loads
+        // above went out.  Otherwise a split is k chunks of 512 tokens (64 per
+        // wave) for every sequence, the smallest k (lane c: c + 1 and c + 65) for
+        // which all sequences' splits fit the slots; the even split's always
+        // does, and stays where no smaller one fits.  Sequence b takes the
+        // slots after those of the sequences before it.
+        const int t_l = (len_l + 511) >> 9;
+        const int t0 = __builtin_amdgcn_readfirstlane(t_l);
+        if (__builtin_amdgcn_ballot_w64(lane < p.B && t_l != t0)) {
+            const int cap = p.B * p.n_splits;
+            const float r1 = 1.0f / (float)(lane + 1), r2 = 1.0f / (float)(lane + 65);
+            int n1 = 0, n2 = 0;
+            for (int i = 0; i < p.B; ++i) {
+                // ceil(t / k) = floor((t + k - 1/2) / k), exact in fp32 while below
+                // 2^12; larger ones stay too large to fit.  At least one.
+                const float t = (float)__builtin_amdgcn_readlane(t_l, i);
+                n1 += max(1, (int)((t + (float)(lane + 1) - 0.5f) * r1));
+                n2 += max(1, (int)((t + (float)(lane + 65) - 0.5f) * r2));
+            }
+            const uint64_t fit1 = __builtin_amdgcn_ballot_w64(n1 <= cap);
+            const uint64_t fit2 = __builtin_amdgcn_ballot_w64(n2 <= cap);
+            const int k = fit1 ? __builtin_ctzll(fit1) + 1 : fit2 ? __builtin_ctzll(fit2) + 65 : 128;
+            if (512 * k < tile_n) {
+                tile_n = 512 * k;
+                wave_tokens = 64 * k;
+                const int n_l = max(1, (t_l + k - 1) / k);
+                int first = 0;
+                for (b = 0; b < p.B; ++b) {
+                    n_splits = __builtin_amdgcn_readlane(n_l, b);
+                    if (u < first + n_splits) break;
+                    first += n_splits;
+                }
+                if (b == p.B) return;                   // no sequence needs this slot
+                sp = u - first;
+                start = sp * tile_n;
+                load_own();
+            }
+        }
+        seq_len = __builtin_amdgcn_readlane(len_l, b);
+        if (sp == 0 && h == 0 && tid == 0) p.slots[b] = make_int2(u, n_splits);
+    } else {
+        seq_len = __builtin_amdgcn_readfirstlane(min(p.seq_lens[b], p.bt_stride * p.block_size));
+    }
+    const int end = min(start + tile_n, seq_len);
+    const int64_t part_row =
+        (FUSED ? (int64_t)u : (int64_t)b * n_splits + sp) * p.H_q + (int64_t)h * GS;
     // This wave's token range: the whole split, or (FUSED) its own share.
-    const int wstart = FUSED ? min(start + wave * p.wave_tokens, end) : start;
-    const int wend = FUSED ? min(wstart + p.wave_tokens, end) : end;
+    const int wstart = FUSED ? min(start + wave * wave_tokens, end) : start;
+    const int wend = FUSED ? min(wstart + wave_tokens, end) : end;
     if (SQK && !*p.k_uniform) {
         // Not the uniform codebook: the output is NaN rather than wrong.
         if (q4 == 0 && r16 < GS) {
@@ -683,7 +742,7 @@ decode_stream_kernel(SplitParams p) {
         for (int i = lane; i < GS * kD; i += 64) p.part_o[part_row * kD + i] = __builtin_nanf("");
         return;
     }
-    if (FUSED && start >= end && p.n_splits == 1) {
+    if (FUSED && start >= end && n_splits == 1) {
         // Empty sequence: the merge of no keys is 0 (weights 0, l clamped).
         for (int i = tid; i < GS * kD; i += kThreads)
             p.out[((int64_t)b * p.H_q + (int64_t)h * GS) * kD + i] = 0;
@@ -1279,7 +1338,7 @@ decode_stream_kernel(SplitParams p) {
                 Ls = fmaf(a, wave_part(w)[GS * kD + GS + g], Ls);
                 Os = fmaf(a, wave_part(w)[g * kD + d], Os);
             }
-            if (p.n_splits == 1) {
+            if (n_splits == 1) {
                 // As the merge's epilogue: fp16(O / l) (attention.py:93).
                 orot[o] = h2f(f2h_after_f32(Os * (1.0f / fmaxf(Ls, 1e-30f))));
             } else {
@@ -1290,7 +1349,7 @@ decode_stream_kernel(SplitParams p) {
                 }
             }
         }
-        if (p.n_splits != 1) return;                     // combine_kernel merges the splits
+        if (n_splits != 1) return;                     // combine_kernel merges the splits
         __syncthreads();
         // out[j] = sum_k fp16(O_rot)[k] * R[j][k], k ascending (compression.py:293-296):
         // thread j reads row j of R once for the group's GS heads.
@@ -1412,10 +1471,12 @@ __device__ __forceinline__ float wave_sum(float v) {
 // 32-lane reduction.  Against R staged in LDS for one wave to walk its rows, a
 // call with several splits takes 1.2-1.4 us less (B=1: N=4K 15.9 -> 14.6 us,
 // N=64K 27.8 -> 26.5).
-template <int HPB>
+// SLOTS: the splits of sequence b are slots[b] = (first, count); one of count 1
+// was written out by its workgroup.
+template <int HPB, bool SLOTS>
 __global__ void __launch_bounds__(256)
 combine_kernel(const float *part_o, const float *part_ml, const float *R, uint16_t *out,
-               int H_q, int n_splits) {
+               int H_q, int n_splits, const int2 *slots) {
     static_assert(HPB == 4 || HPB == 1, "heads per block");
     constexpr int kWph = 4 / HPB;                  // waves per head
     constexpr int kRows = kD / 8;                  // rows of R per thread
@@ -1429,7 +1490,14 @@ combine_kernel(const float *part_o, const float *part_ml, const float *R, uint16
     const int h = h0 + ((HPB == 4) ? wave : 0);
     const int half = lane >> 5, d4 = 4 * (lane & 31);
     const bool live = h < H_q;
-    const int64_t base = (int64_t)b * n_splits * H_q + h;
+    int64_t first = (int64_t)b * n_splits;         // slot of the sequence's first split
+    if constexpr (SLOTS) {
+        const int2 sl = slots[b];
+        if (sl.y == 1) return;
+        first = sl.x;
+        n_splits = sl.y;
+    }
+    const int64_t base = first * H_q + h;
     const float *po = part_o + base * kD + d4;
     const int64_t step = (int64_t)H_q * kD;
     // Empty splits store zeros, so every partial is read unconditionally.
@@ -1547,11 +1615,13 @@ struct WsLayout {
     size_t q_rot, part_o, part_ml, flag, total;
 };
 
-// Plan of the single-launch form: workgroups of one KV head over
-// 8 * wave_tokens tokens (each wave at least one 64-token chunk), about one
-// workgroup per CU over all sequences and heads, at most 4096 pages (64K
-// tokens) per workgroup.  Never more splits than cda_decode_plan's, so its
-// partials fit the same workspace.
+// Plan of the single-launch form: workgroups of one KV head over 8 *
+// wave_tokens tokens, k 64-token chunks per wave (k <= 128: 4096 pages per
+// workgroup), never more splits than cda_decode_plan's, so its partials fit the
+// same workspace.  One workgroup fits a CU, so the grid runs in rounds; k is the
+// one with the least rounds x (k + 3) + 1.5 if a combine follows, in chunks of
+// about 2.5 us: a workgroup's set-up and merge cost about three, the combine
+// one and a half.
 void fused_plan(int B, int H_kv, int max_seq_len, int *wave_tokens, int *n_splits);
 
 WsLayout ws_layout(int B, int H_q, int n_splits) {
@@ -1594,27 +1664,33 @@ int num_cus() {
     return cached;
 }
 
-void fused_plan(int B, int H_kv, int max_seq_len, int *wave_tokens, int *n_splits) {
-    const int n = max_seq_len > 0 ? max_seq_len : 1;
-    const int units = B * H_kv;
-    int s = (num_cus() + units - 1) / units;
-    const int max_by_len = (n + 8 * kStreamPages * 16 - 1) / (8 * kStreamPages * 16);
-    if (s > max_by_len) s = max_by_len;
-    const int min_by_len = (n + 16 * kFusedMaxPages - 1) / (16 * kFusedMaxPages);
-    if (s < min_by_len) s = min_by_len;
-    if (s < 1) s = 1;
-    int wg = (n + s - 1) / s;
-    wg = (wg + 511) / 512 * 512;
-    *wave_tokens = wg / kWaves;
-    *n_splits = (n + wg - 1) / wg;
-}
-
 template <int GS, int L>
 void launch_fused(const SplitParams &p, dim3 grid, hipStream_t st) {
-    if (p.cb_k == p.cb_v)
-        decode_stream_kernel<GS, L, false, true, false><<<grid, kThreads, 0, st>>>(p);
+    const bool one = p.cb_k == p.cb_v;
+    if (one && !p.slots)
+        decode_stream_kernel<GS, L, false, true, false, false><<<grid, kThreads, 0, st>>>(p);
+    else if (one)
+        decode_stream_kernel<GS, L, false, true, false, true><<<grid, kThreads, 0, st>>>(p);
+    else if (!p.slots)
+        decode_stream_kernel<GS, L, false, true, true, false><<<grid, kThreads, 0, st>>>(p);
     else
-        decode_stream_kernel<GS, L, false, true, true><<<grid, kThreads, 0, st>>>(p);
+        decode_stream_kernel<GS, L, false, true, true, true><<<grid, kThreads, 0, st>>>(p);
+}
+
+// Merge and epilogue of n_splits splits a sequence (or those of `slots`): one
+// head per block when four per block would leave CUs idle.
+void launch_combine(const float *part_o, const float *part_ml, const float *R, uint16_t *out, int B,
+                    int H_q, int n_splits, const int2 *slots, hipStream_t st) {
+    const dim3 wide((H_q + 3) / 4, B), narrow(H_q, B);
+    const bool idle = (int64_t)wide.x * B < num_cus();
+    if (idle && slots)
+        combine_kernel<1, true><<<narrow, 256, 0, st>>>(part_o, part_ml, R, out, H_q, n_splits, slots);
+    else if (idle)
+        combine_kernel<1, false><<<narrow, 256, 0, st>>>(part_o, part_ml, R, out, H_q, n_splits, slots);
+    else if (slots)
+        combine_kernel<4, true><<<wide, 256, 0, st>>>(part_o, part_ml, R, out, H_q, n_splits, slots);
+    else
+        combine_kernel<4, false><<<wide, 256, 0, st>>>(part_o, part_ml, R, out, H_q, n_splits, slots);
 }
 
 }  // namespace
@@ -1655,6 +1731,29 @@ extern "C" int cda_decode_plan(int B, int H_q, int H_kv, int max_seq_len, int ti
     if (n_splits_out) *n_splits_out = (n + tn - 1) / tn;
     return CDA_OK;
 }
+
+namespace cda {
+namespace {
+void fused_plan(int B, int H_kv, int max_seq_len, int *wave_tokens, int *n_splits) {
+    const int64_t n = max_seq_len > 0 ? max_seq_len : 1, units = (int64_t)B * H_kv;
+    const int64_t cus = num_cus();
+    int limit = 0;
+    cda_decode_plan(B, H_kv, H_kv, max_seq_len, 0, nullptr, &limit);
+    const int kmax = (int)std::min<int64_t>(16 * kFusedMaxPages / 512, (n + 511) / 512);
+    int64_t best = INT64_MAX;
+    for (int k = kmax; k >= 1; --k) {
+        const int64_t ns = (n + 512 * k - 1) / (512 * k);
+        if (ns > limit && k != kmax) break;
+        const int64_t cost = 2 * ((units * ns + cus - 1) / cus * (k + 3)) + (ns > 1 ? 3 : 0);
+        if (cost < best) {
+            best = cost;
+            *wave_tokens = 64 * k;
+            *n_splits = (int)ns;
+        }
+    }
+}
+}  // namespace
+}  // namespace cda
 
 extern "C" int cda_decode_fused_plan(int B, int H_kv, int max_seq_len, int *wave_tokens_out,
                                      int *n_splits_out) {
@@ -1781,6 +1880,23 @@ int decode_impl(const void *q, const void *kv_cache, int slot_bytes, int H_kv,
         p.out = static_cast<uint16_t *>(out);
         p.wave_tokens = wave_tokens;
         p.bs_shift = (block_size & (block_size - 1)) == 0 ? __builtin_ctz(block_size) : -1;
+        // The slots go by the sequences' lengths where that can pay (up to 64
+        // sequences, one per lane): it shortens a split by some chunks and costs
+        // 0.5 us of set-up and merge, 1 us more where the lengths differ.
+        // Even split / by length: 8 x 4K-16K tokens, 8 KV heads (k = 8 chunks per
+        // wave, 4 splits) 36.0 / 35.0 us, 12 x 8K-30K (30, 2) 105 / 92, 16 x
+        // 4K-16K, 2 KV heads (4, 8) 25.8 / 24.6; but 4 x 4K-16K (4, 8) 26.0 /
+        // 26.6, 8 x 4K-16K, 2 KV heads (2, 16) 18.9 / 19.9, 12 x 1K-4K (4, 2) 24.5
+        // / 25.5, and 16 x 8192, all alike, 4 KV heads (4, 4) 25.3 / 25.8.  (The
+        // kernel's counts are exact below 2^30 tokens; q_rot's part of the
+        // workspace is free here.)
+        const int64_t covered = (int64_t)p.tile_n * nsf;
+        const int k = wave_tokens / 64;
+        const bool by_length = nsf > 1 && B >= 8 && B <= 64 && covered < (1 << 30) &&
+                               (k >= 8 || (k >= 4 && nsf >= 4 && B >= 12));
+        p.B = B;
+        p.max_len = (int)std::min<int64_t>(covered, INT32_MAX);
+        p.slots = by_length ? reinterpret_cast<int2 *>(ws + wf.q_rot) : nullptr;
         const int units = B * nsf;
         p.xcd_map = (units % 8 == 0) ? 1 : 0;
         const dim3 grid(units * H_kv);
@@ -1801,12 +1917,7 @@ int decode_impl(const void *q, const void *kv_cache, int slot_bytes, int H_kv,
         if (g_split_stop && hipEventRecord(g_split_stop, st) != hipSuccess)
             return fail(CDA_E_HIP, f + ": hipEventRecord(stop) failed");
         if (nsf > 1) {
-            if ((int64_t)head_grid.x * B < num_cus())
-                combine_kernel<1><<<dim3(H_q, B), 256, 0, st>>>(p.part_o, p.part_ml, rot_f32,
-                                                                p.out, H_q, nsf);
-            else
-                combine_kernel<4><<<head_grid, 256, 0, st>>>(p.part_o, p.part_ml, rot_f32,
-                                                             p.out, H_q, nsf);
+            launch_combine(p.part_o, p.part_ml, rot_f32, p.out, B, H_q, nsf, p.slots, st);
             CDA_LAUNCH_CHECK("combine_kernel");
         }
         return CDA_OK;
@@ -1882,13 +1993,8 @@ int decode_impl(const void *q, const void *kv_cache, int slot_bytes, int H_kv,
     if (g_split_stop && hipEventRecord(g_split_stop, st) != hipSuccess)
         return fail(CDA_E_HIP, f + ": hipEventRecord(stop) failed");
 
-    // One head per block when four per block would leave CUs idle.
-    if ((int64_t)head_grid.x * B < num_cus())
-        combine_kernel<1><<<dim3(H_q, B), 256, 0, st>>>(p.part_o, p.part_ml, rot_f32,
-                                                        static_cast<uint16_t *>(out), H_q, ns);
-    else
-        combine_kernel<4><<<head_grid, 256, 0, st>>>(p.part_o, p.part_ml, rot_f32,
-                                                     static_cast<uint16_t *>(out), H_q, ns);
+    launch_combine(p.part_o, p.part_ml, rot_f32, static_cast<uint16_t *>(out), B, H_q, ns, nullptr,
+                   st);
     CDA_LAUNCH_CHECK("combine_kernel");
     return CDA_OK;
 }

@@ -441,3 +441,41 @@ def test_decode_single_launch_any_heads_and_slots(gpu, codebooks, name, seq_lens
         _native.set_stream_kernel(True)
     check(fused, case.expected)
     check(fused, general, tol=1e-3)
+
+
+@pytest.mark.parametrize("name,seq_lens,H_kv,gs,levels,slack", [
+    ("one_long", [60000] + [1 + 300 * i for i in range(11)], 1, 4, 16, 0),
+    ("empty_between", [0, 8193, 0, 513, 0, 16385, 512, 0, 4096, 1, 1024, 30000], 1, 8, 16, 0),
+    ("same_chunk_count", [16384 - 40 * i for i in range(12)], 2, 4, 16, 0),
+    ("slack_bound", [900, 33, 2000, 5, 700, 1, 4100, 513], 8, 4, 16, 60000),
+    ("sixty_four", [int(x) for x in np.random.default_rng(12).integers(1, 3000, 63)] + [9000],
+     1, 4, 16, 0),
+    ("k2v2_two_heads", [int(x) for x in np.random.default_rng(13).integers(1, 9000, 15)] + [20000],
+     2, 8, 4, 0),
+    # Beyond 64 sequences, and too short to gain: the even split.
+    ("sixty_five", [int(x) for x in np.random.default_rng(14).integers(1, 900, 64)] + [3000],
+     1, 4, 16, 0),
+    ("short", [3000, 777, 1, 512, 513, 64, 65, 63], 2, 4, 16, 0),
+], ids=lambda v: v if isinstance(v, str) else None)
+def test_decode_slots_by_length(gpu, codebooks, name, seq_lens, H_kv, gs, levels, slack):
+    """Batches of several splits whose slots are dealt by sequence length (up
+    to 64 sequences of different lengths), against the checker and the three
+    launches; twice, bit for bit."""
+    from sub0_amd import _native
+    print(f"[decode-slots] case={name} B={len(seq_lens)} H_kv={H_kv}", flush=True)
+    assert _native.decode_fused_plan(len(seq_lens), H_kv, slack or max(seq_lens))[1] > 1
+    cb = None if levels == 16 else codebooks["lloyd_beta4"].astype(np.float32)
+    case = make_decode_case(7600 + len(name), seq_lens, H_kv=H_kv, gs=gs, cb=cb, fill=0xFF)
+    got = run_gpu_decode(case, gpu, gs=gs, max_seq_len=slack or None)
+    again = run_gpu_decode(case, gpu, gs=gs, max_seq_len=slack or None)
+    _native.set_fused_kernel(False)
+    try:
+        three = run_gpu_decode(case, gpu, gs=gs, max_seq_len=slack or None)
+    finally:
+        _native.set_fused_kernel(True)
+    for b, n in enumerate(seq_lens):
+        if n == 0:
+            assert np.all(got[b] == 0)
+    check(got, case.expected)
+    check(got, three, tol=1e-3)
+    assert np.array_equal(got.view(np.uint16), again.view(np.uint16))
