@@ -79,7 +79,9 @@ constexpr int kKRowDense = kD * 2;                      // 256
 // (ds_read_b64_tr_b16: each 16 lanes read four rows of 16 columns, lane i gets
 // column i): with that order the 8 rows x 64 bytes of one read fall on all 64
 // banks twice.  Passing V through registers into a V^T tile (loads, a 4 x 4
-// transpose, four stores a thread, all between two barriers) took @@.
+// transpose, four stores a thread, all between two barriers) took 1517 us
+// against 1476 (8 prompts of 512-8192 tokens, 32 / 8 heads) and 73.4 against
+// 70.8 (one of 1987).
 
 typedef unsigned v4u32 __attribute__((ext_vector_type(4)));
 
