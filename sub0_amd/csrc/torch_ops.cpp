@@ -136,8 +136,8 @@ void decode_impl(const Tensor &q, const Tensor &kv, const Tensor &bt, const Tens
     TORCH_CHECK_VALUE(bt.size(0) >= B && sl.numel() >= B,
                       "block_table / seq_lens have fewer rows than q");
     const Tensor cb_k = cb_k_in.contiguous();
-    // One tensor for both codebooks lets the single-launch kernel run without
-    // a device-side comparison of the two tables.
+    // One tensor for both codebooks gives the decode kernels one table for K and
+    // V; the three-launch form need not compare two on the device.
     const Tensor cb_v = cb_v_in.data_ptr() == cb_k_in.data_ptr() ? cb_k : cb_v_in.contiguous();
     const size_t need = cda_decode_workspace_size(B, H_q, H_kv, (int)max_seq_len, (int)tile_n);
     Workspace ws = workspace(q, need);
