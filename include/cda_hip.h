@@ -73,6 +73,12 @@ size_t cda_decode_workspace_size(int B, int H_q, int H_kv, int max_seq_len, int 
  * the same shape, so the single launch fits cda_decode_workspace_size(). */
 int cda_decode_fused_plan(int B, int H_kv, int max_seq_len, int *wave_tokens_out,
                           int *n_splits_out);
+/* *by_length_out = 1 where the single-launch decode deals its B * n_splits
+ * slots to the sequences by their lengths (read on the device) instead of
+ * n_splits to each.  A split is then k * 512 tokens for every sequence, the
+ * smallest k for which all splits fit the slots; no sequence gets more than
+ * 1024 splits, the most that the merge takes. */
+int cda_decode_deals_by_length(int B, int H_kv, int max_seq_len, int *by_length_out);
 int cda_decode_full_hmma_v3(const void *q, const void *kv_cache, int64_t num_slots,
                             int slot_bytes, int H_kv, const int32_t *block_table,
                             int bt_stride, const int32_t *seq_lens, const float *cb_k,

@@ -29,6 +29,7 @@ SYMBOLS = (
     "cda_decode_set_timing_events",
     "cda_decode_set_stream_kernel",
     "cda_decode_set_fused_kernel",
+    "cda_decode_deals_by_length",
     "cda_decode_fused_plan",
     "cda_decode_full_hmma_v3_k4v2",
     "cda_paged_encode_fused_k4v2",
@@ -113,6 +114,8 @@ def lib():
         L.cda_decode_fused_plan.restype = _I32
         L.cda_decode_fused_plan.argtypes = [_I32, _I32, _I32, ctypes.POINTER(_I32),
                                             ctypes.POINTER(_I32)]
+        L.cda_decode_deals_by_length.restype = _I32
+        L.cda_decode_deals_by_length.argtypes = [_I32, _I32, _I32, ctypes.POINTER(_I32)]
         L.cda_decode_full_hmma_v3_k4v2.restype = _I32
         L.cda_decode_full_hmma_v3_k4v2.argtypes = [
             _P, _P, _I64, _I32, _I32, _P, _I32, _P, _P, _P, _P, _P, _P,
@@ -220,6 +223,14 @@ def decode_fused_plan(B: int, H_kv: int, max_seq_len: int) -> tuple[int, int]:
     _check(lib().cda_decode_fused_plan(B, H_kv, max_seq_len, ctypes.byref(wt), ctypes.byref(ns)),
            "cda_decode_fused_plan")
     return wt.value, ns.value
+
+
+def decode_deals_by_length(B: int, H_kv: int, max_seq_len: int) -> bool:
+    """True where the single-launch decode deals its slots by sequence length."""
+    on = _I32()
+    _check(lib().cda_decode_deals_by_length(B, H_kv, max_seq_len, ctypes.byref(on)),
+           "cda_decode_deals_by_length")
+    return bool(on.value)
 
 
 def decode_workspace_size(B: int, H_q: int, H_kv: int, max_seq_len: int, tile_n: int = 0) -> int:

@@ -1752,6 +1752,24 @@ void fused_plan(int B, int H_kv, int max_seq_len, int *wave_tokens, int *n_split
         }
     }
 }
+
+// Whether the slots go to the sequences by their lengths: where that can pay
+// (up to 64 sequences, one per lane), as it shortens a split by some chunks and
+// costs 0.5 us of set-up and merge, 1 us more where the lengths differ.
+// Even split / by length: 8 x 4K-16K tokens, 8 KV heads (k = 8 chunks per
+// wave, 4 splits) 36.0 / 35.0 us, 12 x 8K-30K (30, 2) 105 / 92, 16 x
+// 4K-16K, 2 KV heads (4, 8) 25.8 / 24.6; but 4 x 4K-16K (4, 8) 26.0 /
+// 26.6, 8 x 4K-16K, 2 KV heads (2, 16) 18.9 / 19.9, 12 x 1K-4K (4, 2) 24.5
+// / 25.5, and 16 x 8192, all alike, 4 KV heads (4, 4) 25.3 / 25.8.
+// One long sequence among short ones can get every slot but one per other
+// sequence, B * n_splits - (B - 1); the merge holds kMaxSplits, so larger calls
+// keep the even split.  (The kernel's counts are exact below 2^30 tokens.)
+bool deals_by_length(int B, int wave_tokens, int n_splits) {
+    const int k = wave_tokens / 64;
+    return n_splits > 1 && B >= 8 && B <= 64 && B * (n_splits - 1) + 1 <= kMaxSplits &&
+           (int64_t)kWaves * wave_tokens * n_splits < (1 << 30) &&
+           (k >= 8 || (k >= 4 && n_splits >= 4 && B >= 12));
+}
 }  // namespace
 }  // namespace cda
 
@@ -1763,6 +1781,16 @@ extern "C" int cda_decode_fused_plan(int B, int H_kv, int max_seq_len, int *wave
     fused_plan(B, H_kv, max_seq_len, &wt, &ns);
     if (wave_tokens_out) *wave_tokens_out = wt;
     if (n_splits_out) *n_splits_out = ns;
+    return CDA_OK;
+}
+
+extern "C" int cda_decode_deals_by_length(int B, int H_kv, int max_seq_len, int *by_length_out) {
+    if (B <= 0 || H_kv <= 0 || max_seq_len < 0)
+        return fail(CDA_E_INVALID,
+                    "cda_decode_deals_by_length: B, H_kv must be > 0 and max_seq_len >= 0");
+    int wt = 0, ns = 0;
+    fused_plan(B, H_kv, max_seq_len, &wt, &ns);
+    if (by_length_out) *by_length_out = deals_by_length(B, wt, ns) ? 1 : 0;
     return CDA_OK;
 }
 
@@ -1880,23 +1908,12 @@ int decode_impl(const void *q, const void *kv_cache, int slot_bytes, int H_kv,
         p.out = static_cast<uint16_t *>(out);
         p.wave_tokens = wave_tokens;
         p.bs_shift = (block_size & (block_size - 1)) == 0 ? __builtin_ctz(block_size) : -1;
-        // The slots go by the sequences' lengths where that can pay (up to 64
-        // sequences, one per lane): it shortens a split by some chunks and costs
-        // 0.5 us of set-up and merge, 1 us more where the lengths differ.
-        // Even split / by length: 8 x 4K-16K tokens, 8 KV heads (k = 8 chunks per
-        // wave, 4 splits) 36.0 / 35.0 us, 12 x 8K-30K (30, 2) 105 / 92, 16 x
-        // 4K-16K, 2 KV heads (4, 8) 25.8 / 24.6; but 4 x 4K-16K (4, 8) 26.0 /
-        // 26.6, 8 x 4K-16K, 2 KV heads (2, 16) 18.9 / 19.9, 12 x 1K-4K (4, 2) 24.5
-        // / 25.5, and 16 x 8192, all alike, 4 KV heads (4, 4) 25.3 / 25.8.  (The
-        // kernel's counts are exact below 2^30 tokens; q_rot's part of the
-        // workspace is free here.)
         const int64_t covered = (int64_t)p.tile_n * nsf;
-        const int k = wave_tokens / 64;
-        const bool by_length = nsf > 1 && B >= 8 && B <= 64 && covered < (1 << 30) &&
-                               (k >= 8 || (k >= 4 && nsf >= 4 && B >= 12));
         p.B = B;
         p.max_len = (int)std::min<int64_t>(covered, INT32_MAX);
-        p.slots = by_length ? reinterpret_cast<int2 *>(ws + wf.q_rot) : nullptr;
+        // q_rot's part of the workspace is free here.
+        p.slots = deals_by_length(B, wave_tokens, nsf) ? reinterpret_cast<int2 *>(ws + wf.q_rot)
+                                                       : nullptr;
         const int units = B * nsf;
         p.xcd_map = (units % 8 == 0) ? 1 : 0;
         const dim3 grid(units * H_kv);

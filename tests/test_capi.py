@@ -63,6 +63,38 @@ def test_decode_fused_plan_fits_the_workspace():
         _native.decode_fused_plan(0, 8, 100)
 
 
+def test_decode_deal_by_length_fits_the_merge():
+    """Where slots are dealt by length, the deal the kernel makes (the smallest
+    k whose splits of 512 * k tokens fit the B * n_splits slots, if below the
+    even split's) fits them for one long sequence among short ones, and gives
+    no sequence more than the 1024 splits that the merge holds."""
+    from sub0_amd import _native
+    dealt = 0
+    lengths = sorted({(1 << e) + d for e in range(11, 25) for d in (0, 1, 1 << (e - 1))}
+                     | {1440000, 2030000})
+    for H in (1, 2, 4, 8, 16):
+        for B in (8, 9, 12, 16, 23, 32, 48, 63, 64):
+            for n in lengths:
+                if not _native.decode_deals_by_length(B, H, n):
+                    continue
+                dealt += 1
+                wave_tokens, ns = _native.decode_fused_plan(B, H, n)
+                for long in {n, n // 2 + 1025, n // 3, min(n, 512 * (B * ns - B + 1))}:
+                    chunks = [-(-long // 512)] + [1] * (B - 1)
+                    k = next((k for k in range(1, 129)
+                              if sum(max(1, -(-c // k)) for c in chunks) <= B * ns),
+                             wave_tokens // 64)
+                    k = min(k, wave_tokens // 64)
+                    counts = [max(1, -(-c // k)) for c in chunks]
+                    assert sum(counts) <= B * ns, (H, B, n, long, k)
+                    assert max(counts) <= 1024, (H, B, n, long, k, max(counts))
+    assert dealt > 100
+    assert _native.decode_deals_by_length(16, 2, 16384)
+    assert not _native.decode_deals_by_length(65, 1, 65536)     # a lane per sequence
+    with pytest.raises(ValueError):
+        _native.decode_deals_by_length(0, 8, 100)
+
+
 def test_prefill_key_split_plan():
     """Host-side plan of the key-split prefill: split only short chunks over
     long contexts (grid under 256 workgroups, >= 4 key tiles per split, <= 64
