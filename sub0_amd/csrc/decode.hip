@@ -1753,22 +1753,30 @@ void fused_plan(int B, int H_kv, int max_seq_len, int *wave_tokens, int *n_split
     }
 }
 
-// Whether the slots go to the sequences by their lengths: where that can pay
-// (up to 64 sequences, one per lane), as it shortens a split by some chunks and
-// costs 0.5 us of set-up and merge, 1 us more where the lengths differ.
-// Even split / by length: 8 x 4K-16K tokens, 8 KV heads (k = 8 chunks per
-// wave, 4 splits) 36.0 / 35.0 us, 12 x 8K-30K (30, 2) 105 / 92, 16 x
-// 4K-16K, 2 KV heads (4, 8) 25.8 / 24.6; but 4 x 4K-16K (4, 8) 26.0 /
-// 26.6, 8 x 4K-16K, 2 KV heads (2, 16) 18.9 / 19.9, 12 x 1K-4K (4, 2) 24.5
-// / 25.5, and 16 x 8192, all alike, 4 KV heads (4, 4) 25.3 / 25.8.
+// Whether the slots go to the sequences by their lengths (up to 64 sequences,
+// one per lane).  That shortens the longest split by some chunks and costs 0.5 us
+// of set-up and merge, and 1 to 3 us more (8 to 64 sequences) where the lengths
+// differ: it pays for long splits, for many of them, for few sequences.  k =
+// chunks per wave, n = splits.  Time of the even split / by length, geometric
+// mean over calls of 8 to 64 sequences, 1 to 8 KV heads, 144-byte slots, lengths
+// drawn from N/2, N/4 or N/16 up to N (all equal: 0.98 at k = 4-8, 1.00 from 12
+// up):
+//   k >= 16: n = 2 1.08, 3 1.09, 4-7 1.18, 8 up 1.19     12-15: n = 2 1.03, 4 up 1.13
+//   k = 8-11: n = 2 0.98, 3 1.04, 4-7 1.07, 8 up 1.13
+//   k = 6-7: n >= 4: B <= 32 1.06, 48 up 0.98; n = 2 0.96
+//   k = 4-5: n >= 8: B <= 16 1.02, 20-28 1.00, 32 0.95; n = 4-7 0.97
+//   k <= 3: 0.94
 // One long sequence among short ones can get every slot but one per other
 // sequence, B * n_splits - (B - 1); the merge holds kMaxSplits, so larger calls
 // keep the even split.  (The kernel's counts are exact below 2^30 tokens.)
 bool deals_by_length(int B, int wave_tokens, int n_splits) {
     const int k = wave_tokens / 64;
-    return n_splits > 1 && B >= 8 && B <= 64 && B * (n_splits - 1) + 1 <= kMaxSplits &&
-           (int64_t)kWaves * wave_tokens * n_splits < (1 << 30) &&
-           (k >= 8 || (k >= 4 && n_splits >= 4 && B >= 12));
+    if (B < 8 || B > 64 || n_splits < 2 || B * (n_splits - 1) + 1 > kMaxSplits ||
+        (int64_t)kWaves * wave_tokens * n_splits >= (1 << 30))
+        return false;
+    return k >= 8   ? n_splits >= 3 || k >= 12
+           : k >= 6 ? n_splits >= 4 && B <= 32
+                    : k >= 4 && n_splits >= 8 && B <= 16;
 }
 }  // namespace
 }  // namespace cda

@@ -89,7 +89,16 @@ def test_decode_deal_by_length_fits_the_merge():
                     assert sum(counts) <= B * ns, (H, B, n, long, k)
                     assert max(counts) <= 1024, (H, B, n, long, k, max(counts))
     assert dealt > 100
-    assert _native.decode_deals_by_length(16, 2, 16384)
+    # Both sides of the measured line.
+    for B, H, n, plan, on in ((16, 2, 16384, (4, 8), True), (12, 4, 8192, (4, 4), False),
+                              (32, 1, 16384, (4, 8), False), (48, 1, 12288, (5, 5), False),
+                              (12, 4, 12288, (5, 5), False), (12, 1, 60000, (6, 20), True),
+                              (64, 1, 12288, (6, 4), False), (12, 8, 8192, (8, 2), False),
+                              (9, 8, 12288, (8, 3), True), (64, 1, 16384, (8, 4), True),
+                              (12, 8, 16384, (16, 2), True), (8, 2, 16384, (2, 16), False)):
+        wave_tokens, ns = _native.decode_fused_plan(B, H, n)
+        assert (wave_tokens // 64, ns) == plan, (B, H, n)           # chunks per wave, splits
+        assert _native.decode_deals_by_length(B, H, n) is on, (B, H, n)
     assert not _native.decode_deals_by_length(65, 1, 65536)     # a lane per sequence
     with pytest.raises(ValueError):
         _native.decode_deals_by_length(0, 8, 100)
