@@ -87,6 +87,20 @@ int cda_decode_full_hmma_v3(const void *q, const void *kv_cache, int64_t num_slo
                             int block_size, int tile_n, int max_seq_len, float scale,
                             void *workspace, size_t workspace_bytes, void *stream);
 
+/* cda_decode_full_hmma_v3 for a view of a wider table: rows bt_stride entries
+ * apart, of which the first bt_width may be read (a slice of columns; the memory
+ * of the last row can end there).  Entries past seq_lens[b] keys are not used,
+ * but the kernel may read any of the bt_width; cda_decode_full_hmma_v3 may read
+ * any of its (B, bt_stride). */
+int cda_decode_full_hmma_v3_table(const void *q, const void *kv_cache, int64_t num_slots,
+                                  int slot_bytes, int H_kv, const int32_t *block_table,
+                                  int bt_stride, int bt_width, const int32_t *seq_lens,
+                                  const float *cb_k, const float *cb_v, int levels,
+                                  const float *rot_f32, const void *rot_f16, void *out, int B,
+                                  int H_q, int group_size, int block_size, int tile_n,
+                                  int max_seq_len, float scale, void *workspace,
+                                  size_t workspace_bytes, void *stream);
+
 /* The legacy K4V2 cache (cda_attn_v2.py:29: "legacy K4V2 layout (104 B/slot)"):
  * slot = [K codes 4-bit 64 B | V codes 2-bit 32 B | K norm fp32 | V norm fp32],
  * 104 bytes (slot_bytes >= 104, a multiple of 8); cb_k has 16 levels, cb_v 4.

@@ -26,6 +26,7 @@ SYMBOLS = (
     "cda_decode_plan",
     "cda_decode_workspace_size",
     "cda_decode_full_hmma_v3",
+    "cda_decode_full_hmma_v3_table",
     "cda_decode_set_timing_events",
     "cda_decode_set_stream_kernel",
     "cda_decode_set_fused_kernel",
@@ -101,6 +102,10 @@ def lib():
             _I32, _I32, _I32, _I32, _I32, _I32, _F32, _P, _SZ, _P]
         L.cda_decode_noalloc_max_workspace.restype = _SZ
         L.cda_decode_noalloc_max_workspace.argtypes = []
+        L.cda_decode_full_hmma_v3_table.restype = _I32
+        L.cda_decode_full_hmma_v3_table.argtypes = [
+            _P, _P, _I64, _I32, _I32, _P, _I32, _I32, _P, _P, _P, _I32, _P, _P, _P,
+            _I32, _I32, _I32, _I32, _I32, _I32, _F32, _P, _SZ, _P]
         L.cda_decode_full_hmma_v3_noalloc.restype = _I32
         L.cda_decode_full_hmma_v3_noalloc.argtypes = [
             _P, _P, _I64, _I32, _I32, _P, _I32, _P, _P, _P, _I32, _P, _P, _P,
@@ -306,9 +311,9 @@ def decode(q: torch.Tensor, kv_cache: torch.Tensor, block_table: torch.Tensor,
             workspace.numel() - pad, _stream(dev))
         _check(rc, "cda_decode_full_hmma_v3_k4v2")
         return
-    rc = lib().cda_decode_full_hmma_v3(
+    rc = lib().cda_decode_full_hmma_v3_table(
         _ptr(q), _ptr(kv_cache), num_slots, slot_bytes, H_kv, _ptr(block_table),
-        block_table.stride(0), _ptr(seq_lens), _ptr(cb_k), _ptr(cb_v),
+        block_table.stride(0), block_table.shape[1], _ptr(seq_lens), _ptr(cb_k), _ptr(cb_v),
         cb_k.numel(), _ptr(rot_f32), _ptr(rot_f16), _ptr(out), B, H_q, int(group_size),
         int(block_size), int(tile_n), int(max_seq_len), float(scale),
         ctypes.c_void_p(ws_ptr + pad), workspace.numel() - pad, _stream(dev))

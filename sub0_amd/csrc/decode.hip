@@ -70,6 +70,7 @@ struct SplitParams {
     float *part_ml;             // (B, S, H_q, 2): m (log2 domain), l
     int64_t row_bytes;          // H_kv * slot_bytes
     int bt_stride;
+    int bt_width;               // entries of a table row that the caller's memory holds
     int H_q;
     int H_kv;
     int slot_bytes;
@@ -658,7 +659,7 @@ decode_stream_kernel(SplitParams p) {
     };
     // FUSED: every load of the prologue that does not need the sequence length
     // goes out first, so their latencies overlap: the rows of the wave's first
-    // four pages (lane k: page k; the index is clamped to the table row, an
+    // four pages (lane k: page k; the index is clamped to the table row's width, an
     // entry past the sequence is not used), the codebook, q of the head's GQA
     // group and this wave's 16 columns of R.
     constexpr int kQPer = GS * kD / kThreads;             // q values per thread
@@ -669,7 +670,7 @@ decode_stream_kernel(SplitParams p) {
         const int32_t *bt = p.block_table + (int64_t)b * p.bt_stride;
         const int t0 = start + wave * wave_tokens + 16 * (lane & 3);
         const int blk = block_of(t0);
-        first_row = bt[min(blk, p.bt_stride - 1)] * bs + (t0 - blk * bs);
+        first_row = bt[min(blk, p.bt_width - 1)] * bs + (t0 - blk * bs);
 #pragma unroll
         for (int i = 0; i < kQPer; ++i)
             qv[i] = p.q[((int64_t)b * p.H_q + (int64_t)h * GS) * kD + tid + i * kThreads];
@@ -1814,8 +1815,9 @@ namespace {
 // Shared body of the decode entry points.  levels_k / levels_v: 16/16 (K4V4),
 // 4/4 (K2V2) or 16/4 (the legacy K4V2 104-byte slot).
 int decode_impl(const void *q, const void *kv_cache, int slot_bytes, int H_kv,
-                const int32_t *block_table, int bt_stride, const int32_t *seq_lens,
-                const float *cb_k, const float *cb_v, int levels_k, int levels_v,
+                const int32_t *block_table, int bt_stride, int bt_width,
+                const int32_t *seq_lens, const float *cb_k, const float *cb_v, int levels_k,
+                int levels_v,
                 const float *rot_f32, void *out, int B, int H_q, int group_size, int block_size,
                 int tile_n, int max_seq_len, float scale, void *workspace,
                 size_t workspace_bytes, void *stream, const char *fn,
@@ -1835,7 +1837,8 @@ int decode_impl(const void *q, const void *kv_cache, int slot_bytes, int H_kv,
                     "K4V2)");
     CDA_REQUIRE(block_size > 0 && block_size % 16 == 0,
                 f + ": block_size must be a positive multiple of 16");
-    CDA_REQUIRE(max_seq_len >= 0 && bt_stride > 0, f + ": bad max_seq_len / block-table stride");
+    CDA_REQUIRE(max_seq_len >= 0 && bt_stride > 0 && bt_width > 0,
+                f + ": bad max_seq_len / block-table stride or width");
     CDA_REQUIRE((int64_t)16 * H_kv * slot_bytes < (int64_t)1 << 31, f + ": cache row too wide");
     CDA_REQUIRE(((uintptr_t)kv_cache & 15) == 0 && ((uintptr_t)q & 15) == 0,
                 f + ": q and kv_cache must be 16-byte aligned");
@@ -1903,6 +1906,7 @@ int decode_impl(const void *q, const void *kv_cache, int slot_bytes, int H_kv,
         p.part_ml = reinterpret_cast<float *>(ws + wf.part_ml);
         p.row_bytes = (int64_t)H_kv * slot_bytes;
         p.bt_stride = bt_stride;
+        p.bt_width = bt_width;
         p.H_q = H_q;
         p.H_kv = H_kv;
         p.slot_bytes = slot_bytes;
@@ -2026,6 +2030,22 @@ int decode_impl(const void *q, const void *kv_cache, int slot_bytes, int H_kv,
 }  // namespace
 }  // namespace cda
 
+extern "C" int cda_decode_full_hmma_v3_table(
+    const void *q, const void *kv_cache, int64_t num_slots, int slot_bytes, int H_kv,
+    const int32_t *block_table, int bt_stride, int bt_width, const int32_t *seq_lens,
+    const float *cb_k, const float *cb_v, int levels, const float *rot_f32, const void *rot_f16,
+    void *out, int B, int H_q, int group_size, int block_size, int tile_n, int max_seq_len,
+    float scale, void *workspace, size_t workspace_bytes, void *stream) {
+    (void)rot_f16;
+    (void)num_slots;
+    CDA_REQUIRE(levels == 16 || levels == 4,
+                "cda_decode_full_hmma_v3: codebooks must have 16 levels (K4V4) or 4 (K2V2)");
+    return decode_impl(q, kv_cache, slot_bytes, H_kv, block_table, bt_stride, bt_width, seq_lens,
+                       cb_k, cb_v, levels, levels, rot_f32, out, B, H_q, group_size, block_size,
+                       tile_n, max_seq_len, scale, workspace, workspace_bytes, stream,
+                       "cda_decode_full_hmma_v3");
+}
+
 extern "C" int cda_decode_full_hmma_v3(const void *q, const void *kv_cache, int64_t num_slots,
                                        int slot_bytes, int H_kv, const int32_t *block_table,
                                        int bt_stride, const int32_t *seq_lens, const float *cb_k,
@@ -2034,14 +2054,11 @@ extern "C" int cda_decode_full_hmma_v3(const void *q, const void *kv_cache, int6
                                        int group_size, int block_size, int tile_n,
                                        int max_seq_len, float scale, void *workspace,
                                        size_t workspace_bytes, void *stream) {
-    (void)rot_f16;
-    (void)num_slots;
-    CDA_REQUIRE(levels == 16 || levels == 4,
-                "cda_decode_full_hmma_v3: codebooks must have 16 levels (K4V4) or 4 (K2V2)");
-    return decode_impl(q, kv_cache, slot_bytes, H_kv, block_table, bt_stride, seq_lens, cb_k,
-                       cb_v, levels, levels, rot_f32, out, B, H_q, group_size, block_size, tile_n,
-                       max_seq_len, scale, workspace, workspace_bytes, stream,
-                       "cda_decode_full_hmma_v3");
+    return cda_decode_full_hmma_v3_table(q, kv_cache, num_slots, slot_bytes, H_kv, block_table,
+                                         bt_stride, bt_stride, seq_lens, cb_k, cb_v, levels,
+                                         rot_f32, rot_f16, out, B, H_q, group_size, block_size,
+                                         tile_n, max_seq_len, scale, workspace, workspace_bytes,
+                                         stream);
 }
 
 extern "C" int cda_decode_full_hmma_v3_uniform_qk(
@@ -2051,8 +2068,8 @@ extern "C" int cda_decode_full_hmma_v3_uniform_qk(
     int block_size, int tile_n, int max_seq_len, float scale, void *workspace,
     size_t workspace_bytes, void *stream) {
     (void)num_slots;
-    return decode_impl(q, kv_cache, slot_bytes, H_kv, block_table, bt_stride, seq_lens, cb_k,
-                       cb_v, 16, 16, rot_f32, out, B, H_q, group_size, block_size, tile_n,
+    return decode_impl(q, kv_cache, slot_bytes, H_kv, block_table, bt_stride, bt_stride, seq_lens,
+                       cb_k, cb_v, 16, 16, rot_f32, out, B, H_q, group_size, block_size, tile_n,
                        max_seq_len, scale, workspace, workspace_bytes, stream,
                        "cda_decode_full_hmma_v3_uniform_qk", true);
 }
@@ -2068,8 +2085,8 @@ extern "C" int cda_decode_full_hmma_v3_k4v2(const void *q, const void *kv_cache,
                                             size_t workspace_bytes, void *stream) {
     (void)rot_f16;
     (void)num_slots;
-    return decode_impl(q, kv_cache, slot_bytes, H_kv, block_table, bt_stride, seq_lens, cb_k,
-                       cb_v, 16, 4, rot_f32, out, B, H_q, group_size, block_size, tile_n,
+    return decode_impl(q, kv_cache, slot_bytes, H_kv, block_table, bt_stride, bt_stride, seq_lens,
+                       cb_k, cb_v, 16, 4, rot_f32, out, B, H_q, group_size, block_size, tile_n,
                        max_seq_len, scale, workspace, workspace_bytes, stream,
                        "cda_decode_full_hmma_v3_k4v2");
 }

@@ -164,12 +164,11 @@ void decode_impl(const Tensor &q, const Tensor &kv, const Tensor &bt, const Tens
                  "cda_decode_full_hmma_v3_k4v2");
         return;
     }
-    check_rc(cda_decode_full_hmma_v3(q.data_ptr(), kv.data_ptr(), num_slots, slot_bytes, H_kv,
-                                     bt.data_ptr<int32_t>(), (int)bt.stride(0),
-                                     sl.data_ptr<int32_t>(), pk, pv, (int)cb_k.numel(),
-                                     r32.data_ptr<float>(), p16, out.data_ptr(), B, H_q, (int)gs,
-                                     (int)bs, (int)tile_n, (int)max_seq_len, (float)scale, ws.ptr,
-                                     ws.bytes, st),
+    check_rc(cda_decode_full_hmma_v3_table(
+                 q.data_ptr(), kv.data_ptr(), num_slots, slot_bytes, H_kv, bt.data_ptr<int32_t>(),
+                 (int)bt.stride(0), (int)bt.size(1), sl.data_ptr<int32_t>(), pk, pv,
+                 (int)cb_k.numel(), r32.data_ptr<float>(), p16, out.data_ptr(), B, H_q, (int)gs,
+                 (int)bs, (int)tile_n, (int)max_seq_len, (float)scale, ws.ptr, ws.bytes, st),
              "cda_decode_full_hmma_v3");
 }
 

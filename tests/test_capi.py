@@ -176,3 +176,28 @@ def test_python_binding_refuses_cpu_tensors():
         _native.paged_encode(x, x, torch.zeros(4, dtype=torch.int32),
                              torch.zeros(4, 8, 144, dtype=torch.uint8),
                              torch.zeros(16), torch.zeros(16))
+
+
+def test_decode_wrapper_passes_the_table_width(monkeypatch):
+    """A column slice of a block table is handed over with its stride and its
+    width: the single launch reads entries before it knows the lengths, and the
+    slice's last row may end where its memory does."""
+    import torch
+    from sub0_amd import _native
+    calls = {}
+
+    class Recorder:
+        def __getattr__(self, name):
+            return lambda *args: calls.__setitem__(name, args) or 0
+
+    monkeypatch.setattr(_native, "lib", Recorder)
+    monkeypatch.setattr(_native, "_require_gpu", lambda *ts: ts[0].device)
+    monkeypatch.setattr(_native, "_stream", lambda dev: None)
+    q = torch.zeros(3, 32, 128, dtype=torch.float16)
+    cb = torch.zeros(16)
+    table = torch.zeros(3, 20, dtype=torch.int32)[:, 15:]
+    _native.decode(q, torch.zeros(16, 8, 144, dtype=torch.uint8), table,
+                   torch.zeros(3, dtype=torch.int32), cb, cb, torch.zeros(128, 128), None,
+                   torch.zeros_like(q), group_size=4, block_size=16, tile_n=0, max_seq_len=80,
+                   scale=1.0)
+    assert calls["cda_decode_full_hmma_v3_table"][6:8] == (20, 5)

@@ -479,3 +479,62 @@ def test_decode_slots_by_length(gpu, codebooks, name, seq_lens, H_kv, gs, levels
     check(got, case.expected)
     check(got, three, tol=1e-3)
     assert np.array_equal(got.view(np.uint16), again.view(np.uint16))
+
+
+def _table_views(bt):
+    """The block table as slices of wider ones, whose other entries name no page:
+    the first columns, the last (the last row ends with the storage) and, for one
+    row, the tail of a one-dimensional table."""
+    B, W = bt.shape
+    wide = torch.full((B, W + 21), 0x7FFFFFFF, dtype=torch.int32, device=bt.device)
+    first, last = wide.clone()[:, :W], wide.clone()[:, 21:]
+    first.copy_(bt)
+    last.copy_(bt)
+    views = [first, last]
+    if B == 1:
+        flat = wide[0].clone()
+        flat[21:] = bt[0]
+        views.append(flat[None, 21:])
+    return views
+
+
+@pytest.mark.parametrize("name,seq_lens,H_kv,gs,fused", [
+    ("one_row", [77], 8, 4, True),
+    ("one_split", [65] * 33, 8, 4, True),
+    ("splits", [300, 1111, 17], 8, 4, True),
+    ("dealt", [60000] + [1 + 300 * i for i in range(11)], 1, 4, True),
+    ("three_launches", [300, 1111, 17], 8, 4, False),
+    ("general", [300, 1111, 17], 2, 8, False),
+])
+def test_decode_block_table_views(gpu, name, seq_lens, H_kv, gs, fused):
+    """Slices of wider block tables (torch op and ctypes wrapper) give the bits of
+    the contiguous table.  The single launch's early reads stay below the slice's
+    width: waves past the table's end have a short sequence's page to skip."""
+    from sub0_amd import _native
+    from sub0_amd.cda._prebuilt_loader import load_torch_ops_library
+    ops = load_torch_ops_library("cda_hip")
+    print(f"[decode-views] case={name} B={len(seq_lens)} H_kv={H_kv}", flush=True)
+    case = make_decode_case(7700, seq_lens, H_kv=H_kv, gs=gs, fill=0xFF)
+    q, cache, bt, sl, cb, R = (torch.from_numpy(np.ascontiguousarray(x)).to(gpu) for x in (
+        case.q, case.cache, case.block_table, case.seq_lens, case.cb_k, case.R))
+    bound = max(seq_lens)
+    _native.set_fused_kernel(fused)
+    try:
+        want = torch.empty_like(q)
+        _native.decode(q, cache, bt, sl, cb, cb, R, None, want, group_size=gs,
+                       block_size=case.block_size, tile_n=0, max_seq_len=bound,
+                       scale=1 / np.sqrt(128))
+        for view in _table_views(bt):
+            for wrapper in (True, False):
+                out = torch.full_like(q, float("nan"))
+                if wrapper:
+                    _native.decode(q, cache, view, sl, cb, cb, R, None, out, group_size=gs,
+                                   block_size=case.block_size, tile_n=0, max_seq_len=bound,
+                                   scale=1 / np.sqrt(128))
+                else:
+                    ops.decode(q, cache, view, sl, cb, cb, R, R.half(), out, gs, case.block_size,
+                               0, bound, float(1 / np.sqrt(128)))
+                assert torch.equal(out.view(torch.int16), want.view(torch.int16))
+    finally:
+        _native.set_fused_kernel(True)
+    check(want.cpu().numpy(), case.expected)
