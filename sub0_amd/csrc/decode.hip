@@ -528,7 +528,7 @@ template <int N>
 using IC = std::integral_constant<int, N>;
 
 constexpr int kLut2Bytes = 256 * 64 * 4;                   // 64 KiB
-constexpr int kStreamMaxPages = 1024;                      // page rows staged in LDS
+constexpr int kStreamMaxPages = 1024;                      // page ids staged in LDS
 
 typedef unsigned v4u32 __attribute__((ext_vector_type(4)));
 
@@ -565,7 +565,7 @@ constexpr int kStreamRingOff = kLut2Bytes;
 constexpr int kStreamPidOff = kStreamRingOff + kWaves * kStreamPages * kHeadPage;
 constexpr int kStreamLds = kStreamPidOff + kStreamMaxPages * 4;           // 143360 B
 // FUSED form: a workgroup covers up to 4096 pages of one head, and stages q
-// (fp32) and q_rot (fp16) of its GQA group after the page rows.
+// (fp32) and q_rot (fp16) of its GQA group after the page ids.
 constexpr int kFusedMaxPages = 4096;
 constexpr int kFusedQOff = kStreamPidOff + kFusedMaxPages * 4;
 constexpr int kFusedQrOff = kFusedQOff + 8 * kD * 4;
@@ -657,20 +657,26 @@ decode_stream_kernel(SplitParams p) {
     auto block_of = [&](int t) CDA_INLINE {
         return FUSED && p.bs_shift >= 0 ? t >> p.bs_shift : t / bs;
     };
+    // Cache page (16 rows) of token t in block `id`, the sequence's blk-th: pages
+    // count up to 2^35 rows in 32 bits, where rows would end at 2^31 (an 80-byte
+    // slot of one head: 172 GB).
+    auto page_of = [&](int id, int blk, int t) CDA_INLINE {
+        return id * (bs >> 4) + ((t - blk * bs) >> 4);
+    };
     // FUSED: every load of the prologue that does not need the sequence length
-    // goes out first, so their latencies overlap: the rows of the wave's first
+    // goes out first, so their latencies overlap: the ids of the wave's first
     // four pages (lane k: page k; the index is clamped to the table row's width, an
     // entry past the sequence is not used), the codebook, q of the head's GQA
     // group and this wave's 16 columns of R.
     constexpr int kQPer = GS * kD / kThreads;             // q values per thread
-    int first_row = 0;
+    int first_page = 0;
     float cb_lane = 0.0f, rcol[FUSED ? kD / 4 : 1];
     uint16_t qv[FUSED ? kQPer : 1];
     auto load_own = [&]() CDA_INLINE {
         const int32_t *bt = p.block_table + (int64_t)b * p.bt_stride;
         const int t0 = start + wave * wave_tokens + 16 * (lane & 3);
         const int blk = block_of(t0);
-        first_row = bt[min(blk, p.bt_width - 1)] * bs + (t0 - blk * bs);
+        first_page = page_of(bt[min(blk, p.bt_width - 1)], blk, t0);
 #pragma unroll
         for (int i = 0; i < kQPer; ++i)
             qv[i] = p.q[((int64_t)b * p.H_q + (int64_t)h * GS) * kD + tid + i * kThreads];
@@ -776,12 +782,12 @@ decode_stream_kernel(SplitParams p) {
     const int wnpages = (wend - wstart + 15) >> 4;
     const uint32_t ring_w = __builtin_amdgcn_readfirstlane(lds_u32addr(smem)) + kStreamRingOff +
                             wave * (kStreamPages * kHP);
-    int32_t *page_row = reinterpret_cast<int32_t *>(smem + kStreamPidOff);
+    int32_t *page_id = reinterpret_cast<int32_t *>(smem + kStreamPidOff);
     const uint8_t *kv_h = p.kv + (int64_t)h * p.slot_bytes;
     const uint32_t page_bytes = (uint32_t)(16 * row_bytes - h * p.slot_bytes);
-    // DMA of the page starting at cache row row0 into ring slot k.
-    auto issue_row = [&](int64_t row0, int k) CDA_INLINE {
-        const uint64_t base = (uint64_t)(kv_h + row0 * row_bytes);
+    // DMA of cache page `page` into ring slot k.
+    auto issue_page = [&](int page, int k) CDA_INLINE {
+        const uint64_t base = (uint64_t)(kv_h + (int64_t)page * (16 * row_bytes));
         const v4u32 r = {(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)base),
                          (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(base >> 32) & 0xFFFFu),
                          page_bytes, 0x00020000u};
@@ -790,14 +796,14 @@ decode_stream_kernel(SplitParams p) {
         for (int i = 0; i < kDma - 1; ++i) dma_page_chunk(r, src[i], sb + 1024u * i);
         if (lane < 16) dma_page_chunk(r, src[kDma - 1], sb + 1024u * (kDma - 1));
     };
-    // DMA of page t (row from the workgroup's table) into ring slot k.
+    // DMA of page t (id from the workgroup's table) into ring slot k.
     auto issue = [&](int t, int k) CDA_INLINE {
-        issue_row(__builtin_amdgcn_readfirstlane(page_row[wpage0 + t]), k);
+        issue_page(__builtin_amdgcn_readfirstlane(page_id[wpage0 + t]), k);
     };
-    // Cache row of the workgroup's page t.
-    auto row_of = [&](int t) CDA_INLINE {
+    // Cache page of the workgroup's page t.
+    auto id_of = [&](int t) CDA_INLINE {
         const int t0 = start + 16 * t, blk = block_of(t0);
-        return p.block_table[(int64_t)b * p.bt_stride + blk] * bs + (t0 - blk * bs);
+        return page_of(p.block_table[(int64_t)b * p.bt_stride + blk], blk, t0);
     };
     uint4 qb[4];
     // The first chunk's pages go out before the tables are built, so their
@@ -810,13 +816,13 @@ decode_stream_kernel(SplitParams p) {
         for (int m = 0; m < kD / 4; ++m) asm volatile("" : "+v"(rcol[m]));
 #pragma unroll
         for (int k = 0; k < kStreamPages; ++k)
-            if (k < wnpages) issue_row(__builtin_amdgcn_readlane(first_row, k), k);
+            if (k < wnpages) issue_page(__builtin_amdgcn_readlane(first_page, k), k);
     } else {
 #pragma unroll
         for (int k = 0; k < kStreamPages; ++k)
             if (k < wnpages)
-                issue_row(__builtin_amdgcn_readfirstlane(row_of(wpage0 + k)), k);
-        for (int t = tid; t < npages; t += kThreads) page_row[t] = row_of(t);
+                issue_page(__builtin_amdgcn_readfirstlane(id_of(wpage0 + k)), k);
+        for (int t = tid; t < npages; t += kThreads) page_id[t] = id_of(t);
         const uint16_t *qg =
             p.q_rot + ((int64_t)b * p.H_q + (int64_t)h * GS + (r16 & (GS - 1))) * kD + 32 * q4;
 #pragma unroll
@@ -836,7 +842,7 @@ decode_stream_kernel(SplitParams p) {
         a += __shfl_xor(a, 32);
         qsum_neg = -0.9375f * a;
     }
-    int rows[FUSED ? kFusedMaxPages / kThreads : 1];
+    int ids[FUSED ? kFusedMaxPages / kThreads : 1];
     if constexpr (FUSED) {
         // q as fp32, element k = 4m + i of a row at 32i + m: the order in which
         // the lanes of the rotation below take it.
@@ -846,11 +852,11 @@ decode_stream_kernel(SplitParams p) {
             const int o = tid + i * kThreads, k = o & (kD - 1);
             qs[(o & ~(kD - 1)) + (k & 3) * 32 + (k >> 2)] = h2f(qv[i]);
         }
-        // Page rows of the later chunks; stored after the rotation.
+        // Page ids of the later chunks; stored after the rotation.
 #pragma unroll
         for (int i = 0; i < kFusedMaxPages / kThreads; ++i) {
-            rows[i] = 0;
-            if (tid + i * kThreads < npages) rows[i] = row_of(tid + i * kThreads);
+            ids[i] = 0;
+            if (tid + i * kThreads < npages) ids[i] = id_of(tid + i * kThreads);
         }
     }
     {
@@ -902,7 +908,7 @@ decode_stream_kernel(SplitParams p) {
             if (4 * q4 + i < GS) qr[(4 * q4 + i) * kD + 16 * wave + r16] = f2h_after_f32(acc[i]);
 #pragma unroll
         for (int i = 0; i < kFusedMaxPages / kThreads; ++i)
-            if (tid + i * kThreads < npages) page_row[tid + i * kThreads] = rows[i];
+            if (tid + i * kThreads < npages) page_id[tid + i * kThreads] = ids[i];
         __syncthreads();
         const uint16_t *qw = qr + (r16 & (GS - 1)) * kD + 32 * q4;
 #pragma unroll
@@ -1713,7 +1719,7 @@ extern "C" int cda_decode_plan(int B, int H_q, int H_kv, int max_seq_len, int ti
         // One workgroup per CU (the split kernels hold one per CU: their LDS
         // tables are 128-143 KiB), so every split runs in a single round and
         // the per-workgroup set-up is paid once per CU; splits of at least 64
-        // tokens, at most 16384 (the streaming kernel's page-row table) and at
+        // tokens, at most 16384 (the streaming kernel's page table) and at
         // most 512 per sequence.  Measured at B=32, N=64K: 8 splits 527 us,
         // 16: 530, 32: 545, 64: 578.
         const int hg = (H_kv + kWaves - 1) / kWaves;

@@ -538,3 +538,35 @@ def test_decode_block_table_views(gpu, name, seq_lens, H_kv, gs, fused):
     finally:
         _native.set_fused_kernel(True)
     check(want.cpu().numpy(), case.expected)
+
+
+def test_decode_pages_past_2_31_rows(gpu, codebooks):
+    """A one-head K2V2 cache of more than 2^31 rows (172 GB), whose pages the
+    sequences use lie at its end: the bits of the same pages in a small cache.
+    Only those pages are written or read."""
+    from sub0_amd import _native
+    rows = (1 << 31) + (1 << 20)
+    free, _ = torch.cuda.mem_get_info(gpu)
+    if free < rows * 80 + (4 << 30):
+        pytest.skip(f"needs {rows * 80 >> 30} GiB of device memory, {free >> 30} are free")
+    print("[decode-far] cache of 2^31 + 2^20 rows", flush=True)
+    cb4 = codebooks["lloyd_beta4"].astype(np.float32)
+    case = make_decode_case(7800, [700, 33], H_kv=1, gs=4, cb=cb4, fill=0xFF)
+    small = torch.from_numpy(case.cache).to(gpu)
+    bt = torch.from_numpy(case.block_table).to(gpu)
+    q, sl, cb, R = (torch.from_numpy(np.ascontiguousarray(x)).to(gpu)
+                    for x in (case.q, case.seq_lens, case.cb_k, case.R))
+    bs = case.block_size
+    want, got = torch.empty_like(q), torch.empty_like(q)
+    kw = dict(group_size=4, block_size=bs, tile_n=0, max_seq_len=700, scale=1 / np.sqrt(128))
+    _native.decode(q, small, bt, sl, cb, cb, R, None, want, **kw)
+    check(want.cpu().numpy(), case.expected)
+    n = small.shape[0] // bs * bs
+    big = torch.empty(rows, 1, 80, dtype=torch.uint8, device=gpu)
+    try:
+        big[rows - n:].copy_(small[:n])
+        _native.decode(q, big, bt + (rows - n) // bs, sl, cb, cb, R, None, got, **kw)
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    finally:
+        del big
+        torch.cuda.empty_cache()
