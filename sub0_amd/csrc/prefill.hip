@@ -632,9 +632,10 @@ prefill_kernel(PrefillParams p) {
     TileRegs cur;
     TileRows rows_next{0, 0};
     // Dense source: tile j into LDS buffer j & 1 by DMA, two instructions per
-    // wave for K and two for V (keys 8*wave .. +7).  Keys past the end of the
-    // tile's valid range read the last valid key's row (in bounds; their
-    // scores are masked and their weights 0).
+    // wave for K and two for V (keys 8*wave .. +7).  The resource ends with the
+    // tile's last valid key, so the rows past it are not read and come as zeros:
+    // their scores are masked, and the weight 0 times a copy of that key's V
+    // would be NaN where it holds an infinity.
     auto issue_dma = [&](int j) CDA_INLINE {
         if constexpr (!PAGED) {
             const int kb = j * kBN;
@@ -645,7 +646,7 @@ prefill_kernel(PrefillParams p) {
                 const uint64_t base = (uint64_t)(rows + row0);
                 return v4u32{(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)base),
                              (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(base >> 32)) & 0xFFFFu,
-                             (uint32_t)(kBN * pitch), 0x00020000u};
+                             (uint32_t)nk_valid * pitch, 0x00020000u};
             };
             const v4u32 rk = rsrc(p.k_rot), rv = rsrc(p.v_rot);
             const uint32_t dst = __builtin_amdgcn_readfirstlane(lds_addr32(smem)) +
@@ -654,7 +655,7 @@ prefill_kernel(PrefillParams p) {
             for (int t = 0; t < 2; ++t) {
                 const int ins = 2 * wave + t;               // keys 4*ins .. 4*ins + 3
                 const int key = 4 * ins + (lane >> 4);
-                const uint32_t pos = lane & 15, row = (uint32_t)min(key, nk_valid - 1) * pitch;
+                const uint32_t pos = lane & 15, row = (uint32_t)key * pitch;
                 dma_x4_to_lds(rk, row + 16u * (pos ^ (uint32_t)(key & 15)), dst + 1024u * (uint32_t)ins);
                 dma_x4_to_lds(rv, row + 16u * (pos ^ (uint32_t)(4 * (lane >> 4))),
                               dst + kKTile + 1024u * (uint32_t)ins);

@@ -299,3 +299,27 @@ def test_prefill_dense_scratch_matches_bridge(gpu, seq_q, seq_k, H_kv, gs, slack
     out = out.cpu().numpy()
     assert np.array_equal(out.view(np.uint16), bridge.view(np.uint16))
     check(out, case.expected)
+
+
+@pytest.mark.parametrize("seq_k", [[1], [70, 64], [127], [129, 65, 200]])
+def test_dense_prefill_infinite_value(gpu, seq_k):
+    """An infinite coordinate of the last key's V reaches the query that attends
+    the key as that row of the Hadamard matrix times the infinity: the padding of
+    the last key tile carries no copy of it, which would add 0 * Inf = NaN.
+    (Queries that the mask keeps from a key of their tile get its 0 * Inf.)"""
+    print(f"[prefill-inf] seq_k={seq_k}", flush=True)
+    from sub0_amd.cda._prebuilt_loader import load_torch_ops_library
+    ops = load_torch_ops_library("cda_hip")
+    H_kv, gs, T = 2, 4, sum(seq_k)
+    q, k_rot, v_rot = (_dev(synth.normal_f16(6300 + i, (T, h, 128)), gpu)
+                       for i, h in enumerate((H_kv * gs, H_kv, H_kv)))
+    last = np.cumsum(seq_k) - 1
+    v_rot[last, :, 3] = float("inf")
+    cu = _dev(np.concatenate([[0], np.cumsum(seq_k)]).astype(np.int32), gpu)
+    sk = _dev(np.asarray(seq_k, dtype=np.int32), gpu)
+    out = torch.full_like(q, float("nan"))
+    ops.varlen_fwd_hadamard(q, k_rot, v_rot, out, cu, cu, sk, max(seq_k), max(seq_k),
+                            0.25 / np.sqrt(128))
+    got = out.cpu()[last].float()
+    want = torch.from_numpy(np.copysign(np.inf, O.hadamard128()[3])).float()
+    assert torch.equal(got, want.expand_as(got))
