@@ -63,6 +63,47 @@ def test_decode_fused_plan_fits_the_workspace():
         _native.decode_fused_plan(0, 8, 100)
 
 
+def test_decode_fused_plan_is_the_cheapest_and_quick():
+    """The plan's search over round boundaries finds what trying every number of
+    chunks per wave finds (256 CUs; least rounds x (k + 3), in half chunks, 3 for
+    a combine; the largest k of equals), and a long context's plan, made on every
+    call, costs the host no more than a short one's (trying all 128 took 0.8 us
+    at 64K tokens; the least of 40 batches is compared, with 0.4 us allowed)."""
+    import time
+    from sub0_amd import _native
+
+    def every_k(B, H, n):
+        chunks, units, limit = max(1, -(-n // 512)), B * H, _native.decode_plan(B, H, H, n)[1]
+        best = None
+        for k in range(min(128, chunks), 0, -1):
+            ns = -(-chunks // k)
+            if ns > limit and best is not None:
+                break
+            cost = 2 * -(-units * ns // 256) * (k + 3) + (3 if ns > 1 else 0)
+            if best is None or cost < best[0]:
+                best = (cost, 64 * k, ns)
+        return best[1:]
+
+    for B in (1, 2, 3, 5, 8, 12, 16, 31, 33, 64, 65, 257):
+        for H in (1, 2, 3, 8, 16):
+            for n in (0, 1, 512, 513, 1500, 4096, 7000, 16384, 30001, 65536, 100000, 131073,
+                      1000003, 40000000):
+                assert _native.decode_fused_plan(B, H, n) == every_k(B, H, n), (B, H, n)
+
+    L = _native.lib()
+    out = [ctypes.byref(ctypes.c_int32()) for _ in range(2)]
+
+    def host_time(n):
+        best = float("inf")
+        for _ in range(40):
+            t = time.perf_counter()
+            for _ in range(500):
+                L.cda_decode_fused_plan(1, 8, n, *out)
+            best = min(best, time.perf_counter() - t)
+        return best / 500
+    assert host_time(65536) - host_time(512) < 0.4e-6
+
+
 def test_decode_deal_by_length_fits_the_merge():
     """Where slots are dealt by length, the deal the kernel makes (the smallest
     k whose splits of 512 * k tokens fit the B * n_splits slots, if below the
