@@ -1045,15 +1045,26 @@ int launch_prefill(const PrefillParams &p, int B, int max_q, hipStream_t st, con
 // Key-split plan: split only when the unsplit grid leaves CUs idle (fewer
 // than 256 workgroups), into splits of at least 4 key tiles (256 keys), at most
 // kMaxKsplit of them.  One workgroup fits a CU, so a grid runs in rounds of 256;
-// the split count is the one with the least rounds x (tiles per split + 3),
-// a workgroup's set-up and epilogue costing about three tiles.  Rounding the
-// count up to fill 256 workgroups put 80 query blocks in 320 workgroups, two
-// rounds of 20 tiles where three splits run one of 27: 2 x 200-300 queries over
-// 5000 keys, hybrid, 146 -> 106 us a call.
+// the split count is the one with the least rounds x (tiles per split + 3) plus
+// the partials' traffic, in tiles of about 2.1 us: a workgroup's set-up and
+// epilogue cost about three, and 15000 partial rows (one query row of a head and
+// split, 512 B written and read back) about one.  Rounding the count up to fill
+// 256 workgroups put 80 query blocks in 320 workgroups, two rounds of 20 tiles
+// where three splits run one of 27: 2 x 200-300 queries over 5000 keys, hybrid,
+// 146 -> 106 us a call.  Without the traffic term 28 x 64 queries over 10K-16K
+// keys took 8 splits (684 us; unsplit 608, two 645) and 12 x 64 took 8 (283; five
+// 272).  Where the key counts are far below max_k, last splits end early and a
+// grid a little over a round nearly fits it: 12 x 64 over 10K-16K, 3 splits of 86
+// tiles 257 us; 7 x 64, 5 of 52 155 (4 of 65: 167).  With equal counts, which a
+// plan that cannot see them has to expect, the same grids take two full rounds:
+// 16K each, 425 (five: 290) and 262 (four: 175).
 constexpr int kMaxKsplit = 64;
 static_assert(kMaxKsplit <= 64, "prefill_combine_kernel: one lane per split");
 void prefill_ksplit_plan(int B, int H_q, int H_kv, int max_q, int max_k, int *n_split,
-                         int *split_tiles, int max_split = kMaxKsplit) {
+                         int *split_tiles, bool always_merged = false) {
+    // always_merged: the hybrid, whose two parts are merged from partials also
+    // where neither is split, and have half of the merge's splits each.
+    const int max_split = always_merged ? kMaxKsplit / 2 : kMaxKsplit;
     const int qb = 32 * (kWaves / (H_q / H_kv));
     const int64_t wgs = (int64_t)((max_q + qb - 1) / qb) * B * H_kv;
     const int tiles = (max_k + kBN - 1) / kBN;
@@ -1061,10 +1072,13 @@ void prefill_ksplit_plan(int B, int H_q, int H_kv, int max_q, int max_k, int *n_
     *split_tiles = tiles;
     if (wgs <= 0 || wgs >= 256) return;
     constexpr int kFixed = 3;                              // set-up and epilogue, in tiles
-    int64_t best = tiles + kFixed;
+    constexpr int kRowsPerTile = 15000;                    // partial rows moved in a tile's time
+    const int64_t rows = (int64_t)B * max_q * H_q;
+    int64_t best = (int64_t)(tiles + kFixed) * kRowsPerTile + (always_merged ? rows : 0);
     for (int s = 2; s <= std::min(tiles / 4, max_split); ++s) {
         const int per = (tiles + s - 1) / s, ns = (tiles + per - 1) / per;
-        const int64_t cost = (wgs * ns + 255) / 256 * (per + kFixed);
+        const int64_t cost =
+            (wgs * ns + 255) / 256 * (per + kFixed) * kRowsPerTile + ns * rows;
         if (cost < best) {
             best = cost;
             *n_split = ns;
@@ -1489,9 +1503,9 @@ struct HybridPlan {
 HybridPlan hybrid_plan(int B, int T, int H_q, int H_kv, int max_query_len, int max_seq_len) {
     HybridPlan h{};
     prefill_ksplit_plan(B, H_q, H_kv, max_query_len, std::max(1, max_seq_len - 1), &h.na,
-                        &h.na_tiles, kMaxKsplit / 2);
+                        &h.na_tiles, true);
     prefill_ksplit_plan(B, H_q, H_kv, max_query_len, max_query_len, &h.nb, &h.nb_tiles,
-                        kMaxKsplit / 2);
+                        true);
     h.part_bytes = prefill_ws_bytes(T, H_q, h.na + h.nb);
     h.kv_bytes = (((size_t)T * H_kv * kD * 2) + 255) & ~(size_t)255;
     return h;

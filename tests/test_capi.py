@@ -163,6 +163,11 @@ def test_prefill_key_split_plan():
     assert ws(2, 600, 32, 8, 300, 5000) == 3 * 600 * 32 * 128 * 4 + 3 * 600 * 32 * 2 * 4
     # 100 queries x 3 over 4100 keys: 48 workgroups of 65 tiles -> 5 splits of 13.
     assert ws(3, 300, 32, 8, 100, 4100) == 5 * 300 * 32 * 128 * 4 + 5 * 300 * 32 * 2 * 4
+    # The partials' traffic counts: 64 queries x 12 over 16K keys, 96 workgroups
+    # of 257 tiles -> 5 splits of 52 (two rounds), not 8 of 33 (three); x 28, 224
+    # workgroups -> unsplit, not 8 splits.
+    assert ws(12, 768, 32, 8, 64, 16448) == 5 * 768 * 32 * 128 * 4 + 5 * 768 * 32 * 2 * 4
+    assert ws(28, 1792, 32, 8, 64, 16448) == 0
     assert ws(8, 8 * 4096, 32, 8, 4096, 8192) == 0   # config-3-sized grid fills the chip
     assert ws(0, 0, 32, 8, 16, 16384) == 0
     assert ws(1, 16, 32, 5, 16, 16384) == 0          # group size not 4 or 8
