@@ -672,17 +672,20 @@ decode_stream_kernel(SplitParams p) {
     int first_page = 0;
     float cb_lane = 0.0f, rcol[FUSED ? kD / 4 : 1];
     uint16_t qv[FUSED ? kQPer : 1];
-    auto load_own = [&]() CDA_INLINE {
+    auto load_pages = [&]() CDA_INLINE {
         const int32_t *bt = p.block_table + (int64_t)b * p.bt_stride;
         const int t0 = start + wave * wave_tokens + 16 * (lane & 3);
         const int blk = block_of(t0);
         first_page = page_of(bt[min(blk, p.bt_width - 1)], blk, t0);
+    };
+    auto load_q = [&]() CDA_INLINE {
 #pragma unroll
         for (int i = 0; i < kQPer; ++i)
             qv[i] = p.q[((int64_t)b * p.H_q + (int64_t)h * GS) * kD + tid + i * kThreads];
     };
     if constexpr (FUSED) {
-        load_own();
+        load_pages();
+        load_q();
 #pragma unroll
         for (int m = 0; m < kD / 4; ++m)
             rcol[m] = p.R[(4 * m + q4) * kD + 16 * wave + r16];
@@ -726,7 +729,8 @@ decode_stream_kernel(SplitParams p) {
                 if (b == p.B) return;                   // no sequence needs this slot
                 sp = u - first;
                 start = sp * tile_n;
-                load_own();
+                load_pages();
+                load_q();
             }
         }
         seq_len = __builtin_amdgcn_readlane(len_l, b);
@@ -737,9 +741,6 @@ decode_stream_kernel(SplitParams p) {
     const int end = min(start + tile_n, seq_len);
     const int64_t part_row =
         (FUSED ? (int64_t)u : (int64_t)b * n_splits + sp) * p.H_q + (int64_t)h * GS;
-    // This wave's token range: the whole split, or (FUSED) its own share.
-    const int wstart = FUSED ? min(start + wave * wave_tokens, end) : start;
-    const int wend = FUSED ? min(wstart + wave_tokens, end) : end;
     if (SQK && !*p.k_uniform) {
         // Not the uniform codebook: the output is NaN rather than wrong.
         if (q4 == 0 && r16 < GS) {
@@ -764,6 +765,23 @@ decode_stream_kernel(SplitParams p) {
         for (int i = lane; i < GS * kD; i += 64) p.part_o[part_row * kD + i] = 0.0f;
         return;
     }
+
+    if constexpr (FUSED) {
+        // The waves share the tokens that there are, in chunks of 64: a bound far
+        // above the lengths (a captured graph's) would leave them all to the
+        // first wave or two, 6 x 17418 tokens under a bound of 128K, 8 KV heads,
+        // 149 -> 109 us, 24 x 2654 with 512-byte slots 277 -> 86.  Not for one
+        // chunk less, which the second read of the table row costs; marked unlikely,
+        // or one chunk per wave takes 0.3 us more (8 queries per head, 895 tokens 16.4).
+        const int share = ((end - start + 64 * kWaves - 1) / (64 * kWaves)) * 64;
+        if (__builtin_expect(wave_tokens > 128 && share + 128 <= wave_tokens, 0)) {
+            wave_tokens = share;
+            load_pages();
+        }
+    }
+    // This wave's token range: the whole split, or (FUSED) its own share.
+    const int wstart = FUSED ? min(start + wave * wave_tokens, end) : start;
+    const int wend = FUSED ? min(wstart + wave_tokens, end) : end;
 
     // Source offset of this lane's piece of each DMA instruction within the
     // head's page rows: piece 64 * i + lane of the page's 16 * kPieces.

@@ -570,3 +570,60 @@ def test_decode_pages_past_2_31_rows(gpu, codebooks):
     finally:
         del big
         torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("name,seq_lens,H_kv,gs,levels,slot", [
+    ("one_split", [2654] * 4, 8, 4, 16, 144),
+    ("chunk_edges", [511, 512, 513, 1024, 1025, 1, 0, 64], 8, 4, 16, 144),
+    ("last_split_short", [40000, 16385, 8193], 2, 8, 16, 160),
+    ("k2v2_dealt", [int(x) for x in np.random.default_rng(15).integers(0, 6000, 12)], 8, 8, 4, 80),
+])
+def test_decode_under_a_loose_bound(gpu, codebooks, name, seq_lens, H_kv, gs, levels, slot):
+    """Lengths far below max_seq_len (131072), where the waves of a workgroup
+    share what there is instead of their part of the bound: the checker's output,
+    and the tight bound's."""
+    print(f"[decode-loose] case={name} B={len(seq_lens)} H_kv={H_kv}", flush=True)
+    cb = None if levels == 16 else codebooks["lloyd_beta4"].astype(np.float32)
+    case = make_decode_case(7700 + len(name), seq_lens, H_kv=H_kv, gs=gs, cb=cb, fill=0xFF)
+    pad = slot - case.cache.shape[-1]
+    case.cache = np.pad(case.cache, ((0, 0), (0, 0), (0, pad)), constant_values=0xFF)
+    loose = run_gpu_decode(case, gpu, gs=gs, max_seq_len=131072)
+    check(loose, case.expected)
+    for b, n in enumerate(seq_lens):
+        if n == 0:
+            assert np.all(loose[b] == 0)
+
+
+def test_decode_loose_bound_is_not_far_slower(gpu):
+    """24 sequences of 2654 tokens, 512-byte slots, under a bound of 131072: the
+    work is the tight bound's, and a call took nine times as long where one
+    wave of eight had it all.  Four times is allowed."""
+    from sub0_amd import _native
+    B, n, H = 24, 2654, 8
+    g = torch.Generator(device=gpu).manual_seed(3)
+    w = (n + 15) // 16
+    cache = torch.randint(0, 256, (B * w * 16, H, 512), dtype=torch.uint8, device=gpu, generator=g)
+    cache[..., 128:136] = torch.ones(2, device=gpu).view(torch.uint8)
+    bt = torch.arange(B * w, dtype=torch.int32, device=gpu).view(B, w)
+    q = torch.randn(B, 4 * H, 128, device=gpu, generator=g).half()
+    cb = torch.linspace(-0.2, 0.2, 16, device=gpu)
+    R = torch.eye(128, device=gpu)
+    out = torch.empty_like(q)
+    lens = torch.full((B,), n, dtype=torch.int32, device=gpu)
+
+    def us(bound):
+        times = []
+        for _ in range(7):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            torch.cuda._sleep(1000000)
+            a.record()
+            for _ in range(10):
+                _native.decode(q, cache, bt, lens, cb, cb, R, None, out, group_size=4,
+                               block_size=16, tile_n=0, max_seq_len=bound, scale=0.09)
+            b.record()
+            torch.cuda.synchronize()
+            times.append(a.elapsed_time(b) * 100)
+        return sorted(times)[3]
+    tight, loose = us(n), us(131072)
+    print(f"[decode-loose] tight {tight:.1f} us, loose {loose:.1f} us", flush=True)
+    assert loose < 4 * tight
