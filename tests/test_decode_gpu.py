@@ -597,7 +597,8 @@ def test_decode_under_a_loose_bound(gpu, codebooks, name, seq_lens, H_kv, gs, le
 def test_decode_loose_bound_is_not_far_slower(gpu):
     """24 sequences of 2654 tokens, 512-byte slots, under a bound of 131072: the
     work is the tight bound's, and a call took nine times as long where one
-    wave of eight had it all.  Four times is allowed."""
+    wave of eight had it all, 2.7 times where two XCDs of eight did.  Twice is
+    allowed."""
     from sub0_amd import _native
     B, n, H = 24, 2654, 8
     g = torch.Generator(device=gpu).manual_seed(3)
@@ -626,4 +627,4 @@ def test_decode_loose_bound_is_not_far_slower(gpu):
         return sorted(times)[3]
     tight, loose = us(n), us(131072)
     print(f"[decode-loose] tight {tight:.1f} us, loose {loose:.1f} us", flush=True)
-    assert loose < 4 * tight
+    assert loose < 2 * tight
