@@ -1,4 +1,4 @@
-// Library-wide C ABI pieces: version and per-thread error text.
+// Library-wide pieces: version, per-thread error text, the device's CU count.
 #include "cda_common.h"
 
 namespace cda {
@@ -8,6 +8,17 @@ thread_local std::string g_last_error;
 }
 
 void set_error(const std::string &msg) { g_last_error = msg; }
+
+int num_cus() {
+    static const int cus = [] {
+        int dev = 0, n = 0;
+        return hipGetDevice(&dev) == hipSuccess &&
+                       hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) ==
+                           hipSuccess && n > 0
+                   ? n : 256;
+    }();
+    return cus;
+}
 
 }  // namespace cda
 

@@ -20,6 +20,9 @@ inline int fail(int code, const std::string &msg) {
     return code;
 }
 
+// CUs of the first device that a plan was made for (256 without one).
+int num_cus();
+
 #define CDA_REQUIRE(cond, msg)                                               \
     do {                                                                     \
         if (!(cond)) return ::cda::fail(CDA_E_INVALID, std::string(msg));    \

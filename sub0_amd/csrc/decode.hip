@@ -1682,20 +1682,6 @@ std::atomic<bool> g_allow_stream{true};
 // form also applies.
 std::atomic<bool> g_allow_fused{true};
 
-int num_cus() {
-    static int cached = 0;
-    if (!cached) {
-        int dev = 0, n = 0;
-        if (hipGetDevice(&dev) == hipSuccess &&
-            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
-            n > 0)
-            cached = n;
-        else
-            cached = 256;
-    }
-    return cached;
-}
-
 template <int GS, int L>
 void launch_fused(const SplitParams &p, dim3 grid, hipStream_t st) {
     const bool one = p.cb_k == p.cb_v;

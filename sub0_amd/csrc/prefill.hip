@@ -1042,13 +1042,13 @@ int launch_prefill(const PrefillParams &p, int B, int max_q, hipStream_t st, con
     return launch_combine(p, p.n_ksplit, B, st, fn);
 }
 
-// Key-split plan: split only when the unsplit grid leaves CUs idle (fewer
-// than 256 workgroups), into splits of at least 4 key tiles (256 keys), at most
-// kMaxKsplit of them.  One workgroup fits a CU, so a grid runs in rounds of 256;
-// the split count is the one with the least rounds x (tiles per split + 3) plus
-// the partials' traffic, in tiles of about 2.1 us: a workgroup's set-up and
-// epilogue cost about three, and 15000 partial rows (one query row of a head and
-// split, 512 B written and read back) about one.  Rounding the count up to fill
+// Key-split plan: split only when the unsplit grid leaves CUs idle, into
+// splits of at least 4 key tiles (256 keys), at most kMaxKsplit of them.  One
+// workgroup fits a CU, so a grid runs in rounds of as many; the split count is the
+// one with the least rounds x (tiles per split + 3) plus the partials' traffic, in
+// tiles of about 2.1 us: a workgroup's set-up and epilogue cost about three, and
+// 15000 partial rows (one query row of a head and split, 512 B written and read
+// back) about one.  Of 256 CUs (MI355X): rounding the count up to fill
 // 256 workgroups put 80 query blocks in 320 workgroups, two rounds of 20 tiles
 // where three splits run one of 27: 2 x 200-300 queries over 5000 keys, hybrid,
 // 146 -> 106 us a call.  Without the traffic term 28 x 64 queries over 10K-16K
@@ -1057,7 +1057,9 @@ int launch_prefill(const PrefillParams &p, int B, int max_q, hipStream_t st, con
 // grid a little over a round nearly fits it: 12 x 64 over 10K-16K, 3 splits of 86
 // tiles 257 us; 7 x 64, 5 of 52 155 (4 of 65: 167).  With equal counts, which a
 // plan that cannot see them has to expect, the same grids take two full rounds:
-// 16K each, 425 (five: 290) and 262 (four: 175).
+// 16K each, 425 (five: 290) and 262 (four: 175).  Nor can it see query counts:
+// 3 x 194-389 queries over 2.5K-4K, hybrid, 144 workgroups of which 128 have
+// queries, take 3 splits (153 us) where 2 fit one round (135).
 constexpr int kMaxKsplit = 64;
 static_assert(kMaxKsplit <= 64, "prefill_combine_kernel: one lane per split");
 void prefill_ksplit_plan(int B, int H_q, int H_kv, int max_q, int max_k, int *n_split,
@@ -1070,7 +1072,8 @@ void prefill_ksplit_plan(int B, int H_q, int H_kv, int max_q, int max_k, int *n_
     const int tiles = (max_k + kBN - 1) / kBN;
     *n_split = 1;
     *split_tiles = tiles;
-    if (wgs <= 0 || wgs >= 256) return;
+    const int64_t cus = num_cus();
+    if (wgs <= 0 || wgs >= cus) return;
     constexpr int kFixed = 3;                              // set-up and epilogue, in tiles
     constexpr int kRowsPerTile = 15000;                    // partial rows moved in a tile's time
     const int64_t rows = (int64_t)B * max_q * H_q;
@@ -1078,7 +1081,7 @@ void prefill_ksplit_plan(int B, int H_q, int H_kv, int max_q, int max_k, int *n_
     for (int s = 2; s <= std::min(tiles / 4, max_split); ++s) {
         const int per = (tiles + s - 1) / s, ns = (tiles + per - 1) / per;
         const int64_t cost =
-            (wgs * ns + 255) / 256 * (per + kFixed) * kRowsPerTile + ns * rows;
+            (wgs * ns + cus - 1) / cus * (per + kFixed) * kRowsPerTile + ns * rows;
         if (cost < best) {
             best = cost;
             *n_split = ns;
