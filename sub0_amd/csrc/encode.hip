@@ -71,7 +71,6 @@ struct EncodeParams {
     const float *cb_v;
 };
 
-
 constexpr int kEncWaves = 4;          // waves 2q, 2q+1: K and V of item group q
 
 // Ordered-integer image of an fp32 value (monotone in the value; -0 < +0).
@@ -95,14 +94,16 @@ __device__ __forceinline__ bool pick_upper(float u, float lo, float hi) {
 // Thresholds at or below -1 always hold after the clamp (beta = -inf);
 // thresholds above 1 never do (beta = +inf).
 //
-// K lanes (j = 0..K-1, aligned in the wave) search one threshold together: each
-// tests one of K points, which cuts the interval of ordered bit patterns by K a
-// turn, 8 turns for K = 16 or 11 for K = 8 where one lane's bisection took 31
-// (2.5 us before the first vector could be quantised).  Every lane of the wave
-// has to call; those without a threshold pass live = false.
-template <int K>
+// kSearch lanes (j = 0..7, aligned in the wave) search one threshold together:
+// each tests one of eight points, which cuts the interval of ordered bit patterns
+// by eight a turn, 11 turns where one lane's bisection took 31 (2.5 us before the
+// first vector could be quantised).  Every lane of the wave has to call; those
+// without a threshold pass live = false.
+constexpr int kSearch = 64 * kEncWaves / 32;          // a block's lanes, 16 thresholds a role
+static_assert(kSearch == 8, "lanes per threshold");
 __device__ void codebook_threshold(const float *cb, int i, int j, bool live, double *beta,
                                    int *strict) {
+    constexpr int K = kSearch;
     const float lo = live ? cb[i - 1] : 0.0f, hi = live ? cb[i] : 0.0f;
     uint32_t a = f2key(lo) + 1u, b = f2key(hi);
     // The answer lies in [a, b].  The largest point tested is never below b,
@@ -136,13 +137,13 @@ __device__ void codebook_threshold(const float *cb, int i, int j, bool live, dou
 template <int LK, int LV>
 __device__ __forceinline__ void codebook_thresholds(const EncodeParams &p, double (&beta)[2][16],
                                                     int (&strict)[2][16], float (&s_cb)[2][16]) {
-    constexpr int K = 64 * kEncWaves / 32;            // lanes per threshold: 32 of the two roles
+    constexpr int K = kSearch;
     const int at = (int)threadIdx.x / K, r = at >> 4, i = at & 15;
     const float *cb = r ? p.cb_v : p.cb_k;
     const int j = (int)threadIdx.x & (K - 1);
     const bool in = i < (r ? LV : LK);
     if (in && j == 0) s_cb[r][i] = cb[i];
-    codebook_threshold<K>(cb, i, j, in && i > 0, &beta[r][i], &strict[r][i]);
+    codebook_threshold(cb, i, j, in && i > 0, &beta[r][i], &strict[r][i]);
 }
 
 // Smallest fp32 >= t (t finite or infinite).
@@ -437,39 +438,33 @@ paged_encode_kernel(EncodeParams p) {
     else finish(std::integral_constant<int, LV>{});
 }
 
-// Small batches: P = 16 lanes share a vector, and lane r of them runs the chains
-// of outputs r + 16m as a tree of fp32 fmas (688 a lane).  That ends sooner than
-// the 172 MFMAs of a wave above while a SIMD has only a wave or two to run.
-template <int P>
-struct EncLayout {
-    static constexpr int V = 64 / P;          // vectors per wave
-    static constexpr int M = kD / P;          // outputs per lane
-    static constexpr int kPitch = kD + P;     // floats per vector row in LDS (bank spread)
-    // per wave: V rows of sq / idx, then V x 16 thresholds, V x 8 lane sums
-    static constexpr int kThrPitch = 17;      // thresholds per vector (bank spread)
-    static constexpr int kWaveFloats = V * kPitch + V * kThrPitch + V * 8;
-};
+// Small batches: 16 lanes share a vector, and lane r of them runs the chains of
+// outputs r + 16m as a tree of fp32 fmas (688 a lane).  That ends sooner than the
+// 172 MFMAs of a wave above while a SIMD has only a wave or two to run.
+constexpr int kSmallLanes = 16;               // per vector
+constexpr int kSmallVecs = 64 / kSmallLanes;  // vectors per wave
+constexpr int kSmallPitch = kD + kSmallLanes; // floats per vector row in LDS (bank spread)
 
-template <int LK, int LV, int P>
+template <int LK, int LV>
 __global__ void __launch_bounds__(64 * kEncWaves)
 paged_encode_small_kernel(EncodeParams p) {
-    using Lay = EncLayout<P>;
-    constexpr int V = Lay::V, M = Lay::M, PITCH = Lay::kPitch;
+    constexpr int P = kSmallLanes, V = kSmallVecs, M = kD / P;   // M: outputs per lane
     // Slot: [K codes KBK | V codes KBV | K norm | V norm | pad].
     constexpr int KBK = kD * (LK == 16 ? 4 : 2) / 8;
     constexpr int KBV = kD * (LV == 16 ? 4 : 2) / 8;
     __shared__ double s_beta[2][16];
     __shared__ int s_strict[2][16];
     __shared__ float s_cb[2][16];
-    __shared__ float s_w[kEncWaves][Lay::kWaveFloats];
+    // Per wave: V rows of sq / idx, then V x 16 thresholds, V x 8 lane sums.
+    __shared__ __align__(16) float s_w[kEncWaves][V * (kSmallPitch + kThrPitch + 8)];
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int role = wave & 1;                        // wave-uniform: 0 = K, 1 = V
     const int g = lane / P, r = lane % P;
-    float *sq_row = s_w[wave] + g * PITCH;            // this vector's 128 floats
-    float *thr = s_w[wave] + V * PITCH + g * Lay::kThrPitch;
-    float *lsum = s_w[wave] + V * PITCH + V * Lay::kThrPitch + g * 8;
+    float *sq_row = s_w[wave] + g * kSmallPitch;      // this vector's 128 floats
+    float *thr = s_w[wave] + V * kSmallPitch + g * kThrPitch;
+    float *lsum = s_w[wave] + V * (kSmallPitch + kThrPitch) + g * 8;
 
     // (token, head) item of this lane group; fewer than 2^31 items (host check).
     const uint32_t items = (uint32_t)(p.num_tokens * p.H_kv);
@@ -481,7 +476,7 @@ paged_encode_small_kernel(EncodeParams p) {
     const int64_t t = t32;
 
     // ---- load the vector (lanes past the last item read the first and store
-    // nothing; all P lanes of the group read the same 256 B) ----
+    // nothing; the 16 lanes of a vector read the same 256 B) ----
     // Kept as packed fp16 pairs; each x_k is widened to fp32 once, where the
     // chains use it (xf below).
     uint32_t xw[kD / 2];
@@ -555,15 +550,11 @@ paged_encode_small_kernel(EncodeParams p) {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    if (r < 8) {
+        float a = sq_row[r];
 #pragma unroll
-    for (int l0 = 0; l0 < 8; l0 += P) {
-        const int l = l0 + r;
-        if (l < 8) {
-            float a = sq_row[l];
-#pragma unroll
-            for (int c = 1; c < kD / 8; ++c) a = __fadd_rn(a, sq_row[8 * c + l]);
-            lsum[l] = a;
-        }
+        for (int c = 1; c < kD / 8; ++c) a = __fadd_rn(a, sq_row[8 * c + r]);
+        lsum[r] = a;
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -578,19 +569,14 @@ paged_encode_small_kernel(EncodeParams p) {
     // codebook (K: LK levels, V: LV levels; wave-uniform branch).
     auto finish = [&](auto levels) CDA_INLINE {
         constexpr int L = decltype(levels)::value;
-        constexpr int KB = kD * (L == 16 ? 4 : 2) / 8;   // code bytes of this role
         // ---- per-vector thresholds in the x domain ------------------------------
         const bool finite_n = fabsf(n) < __builtin_inff();
-    #pragma unroll
-        for (int i0 = 1; i0 < L; i0 += P) {
-            const int i = i0 + r;
-            if (i < L) {
-                const double beta = s_beta[role][i];
-                double tt = (double)n * beta;             // exact: 24 x 25 significant bits
-                if (s_strict[role][i] && finite_n) tt = next_up(tt);
-                const float th = round_up_f32(tt);
-                thr[thr_pos<L>(i)] = th == 0.0f ? -0.0f : th;
-            }
+        if (r > 0 && r < L) {                             // lane r: threshold r
+            const double beta = s_beta[role][r];
+            double tt = (double)n * beta;                 // exact: 24 x 25 significant bits
+            if (s_strict[role][r] && finite_n) tt = next_up(tt);
+            const float th = round_up_f32(tt);
+            thr[thr_pos<L>(r)] = th == 0.0f ? -0.0f : th;
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -622,35 +608,20 @@ paged_encode_small_kernel(EncodeParams p) {
         if (slot < 0 || slot >= p.num_slots) return;
         uint8_t *dst = p.cache + slot * p.row_bytes + (int64_t)h * p.slot_bytes;
         uint8_t *codes = dst + (role ? KBK : 0);
-        // Lane r packs code bytes [r * KB / P, (r + 1) * KB / P).
-        constexpr int BPL = KB / P;                        // bytes per lane: 16/4 (K4) or 8/2 (K2)
-        constexpr int EPB = L == 16 ? 2 : 4;               // elements per byte
-        const uint32_t *src = reinterpret_cast<const uint32_t *>(idx_row + r * BPL * EPB);
-        uint32_t packed[(BPL + 3) / 4];
+        // Lane r packs the codes of dims [8r, 8r + 8): four bytes of 4-bit codes,
+        // two of 2-bit codes.
+        const uint2 e = *reinterpret_cast<const uint2 *>(idx_row + 8 * r);
+        auto code_at = [&](int i) CDA_INLINE { return ((i < 4 ? e.x : e.y) >> (8 * (i & 3))) & 0xFFu; };
+        uint32_t packed = 0;
     #pragma unroll
-        for (int w = 0; w < (BPL + 3) / 4; ++w) packed[w] = 0;
-    #pragma unroll
-        for (int b = 0; b < BPL; ++b) {
-            uint32_t byte;
-            if constexpr (L == 16) {
-                const uint32_t e = src[b / 2] >> (16 * (b & 1));      // elements 2b, 2b+1
-                byte = ((e & 0xFu) << 4) | ((e >> 8) & 0xFu);
-            } else {
-                const uint32_t e = src[b];                           // elements 4b .. 4b+3
-                byte = ((e & 3u) << 6) | (((e >> 8) & 3u) << 4) | (((e >> 16) & 3u) << 2) |
-                       ((e >> 24) & 3u);
-            }
-            packed[b / 4] |= byte << (8 * (b & 3));
-        }
-        if constexpr (BPL >= 4) {
-    #pragma unroll
-            for (int w = 0; w < BPL / 4; ++w)
-                reinterpret_cast<uint32_t *>(codes + r * BPL)[w] = packed[w];
-        } else {
-            *reinterpret_cast<uint16_t *>(codes + r * BPL) = (uint16_t)packed[0];
-        }
+        for (int i = 0; i < 8; ++i)
+            packed |= L == 16 ? code_at(i) << (8 * (i / 2) + 4 * (1 - i % 2))
+                              : code_at(i) << (8 * (i / 4) + 2 * (3 - i % 4));
+        if constexpr (L == 16)
+            reinterpret_cast<uint32_t *>(codes)[r] = packed;
+        else
+            reinterpret_cast<uint16_t *>(codes)[r] = (uint16_t)packed;
         if (r == 0) *reinterpret_cast<float *>(dst + KBK + KBV + 4 * role) = n;
-
     };
     if (role == 0) finish(std::integral_constant<int, LK>{});
     else finish(std::integral_constant<int, LV>{});
@@ -664,8 +635,8 @@ constexpr int64_t kSmallItems = 4096;
 template <int LK, int LV>
 void launch_encode(const EncodeParams &p, int64_t items, hipStream_t st) {
     if (items <= kSmallItems) {
-        constexpr int per_block = (64 / 16) * kEncWaves / 2;
-        paged_encode_small_kernel<LK, LV, 16>
+        constexpr int per_block = kSmallVecs * kEncWaves / 2;
+        paged_encode_small_kernel<LK, LV>
             <<<dim3((unsigned)((items + per_block - 1) / per_block)), 64 * kEncWaves, 0, st>>>(p);
     } else {
         constexpr int per_block = 16 * kEncWaves / 2;
