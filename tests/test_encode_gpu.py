@@ -192,3 +192,37 @@ def test_encode_mfma_form_edges(gpu, codebooks, levels, T, H_kv):
     got = run_gpu_encode(gpu, k, v, slots, cb_k, T + 9, sb, 0x3C, cb_v=cb_v)
     bad = np.argwhere(got != exp)
     assert bad.size == 0, f"{len(bad)} mismatching bytes, first {bad[:5].tolist()}"
+
+
+@pytest.mark.parametrize("levels,T,H_kv", [(16, 40, 8), (16, 700, 8), (4, 1367, 3)])
+def test_encode_non_finite_vectors(gpu, codebooks, levels, T, H_kv):
+    """Vectors with infinities and NaNs among finite ones, in the 16-lane form
+    (40 tokens) and the MFMA form: the checker's codes for all of them, its norm
+    bits for the finite ones, also beside a non-finite one in the same wave, and
+    its infinite or NaN norm for the others."""
+    print(f"[encode] non-finite levels={levels} T={T} H_kv={H_kv}", flush=True)
+    cb = codebooks["lloyd_beta16" if levels == 16 else "lloyd_beta4"]
+    k = synth.kv_with_outliers(531, (T, H_kv, 128))
+    v = synth.normal_f16(532, (T, H_kv, 128))
+    bad_k, bad_v = np.zeros((T, H_kv), bool), np.zeros((T, H_kv), bool)
+    for x, bad, first in ((k, bad_k, 1), (v, bad_v, 2)):
+        for j, t in enumerate(range(first, T, 11)):
+            x[t, j % H_kv, (7 * j) % 128] = (np.inf, -np.inf, np.nan)[j % 3]
+            bad[t, j % H_kv] = True
+        x[first + 3, 0] = np.inf
+        bad[first + 3, 0] = True
+    slots = synth.permuted_block_table(533, 1, T + 9)[0][:T].astype(np.int64)
+    sb = 144 if levels == 16 else 80
+    kb = 64 if levels == 16 else 32
+    got = run_gpu_encode(gpu, k, v, slots, cb, T + 9, sb, 0x3C)
+    with np.errstate(all="ignore"):
+        exp = expected_cache(k, v, slots, cb, T + 9, sb, 0x3C)
+    for role, bad in ((0, bad_k), (1, bad_v)):
+        codes = slice(role * kb, (role + 1) * kb)
+        norm = slice(2 * kb + 4 * role, 2 * kb + 4 * role + 4)
+        g, e = got[slots], exp[slots]
+        assert np.array_equal(g[..., codes], e[..., codes])
+        assert np.array_equal(g[~bad][:, norm], e[~bad][:, norm])
+        ng, ne = (np.ascontiguousarray(a[bad][:, norm]).view(np.float32)[:, 0] for a in (g, e))
+        assert not np.isfinite(ng).any()
+        assert np.array_equal(ng, ne, equal_nan=True)
