@@ -254,15 +254,12 @@ __device__ __forceinline__ int block_of(const PrefillParams &p, int kpos) {
     return p.bs_shift >= 0 ? (kpos >> p.bs_shift) : (kpos / p.block_size);
 }
 
-template <bool PAGED>
 __device__ __forceinline__ TileRows fetch_rows(const PrefillParams &p, const int32_t *bt_row,
                                                int kbase, int nk_valid, int tid) {
     TileRows r{0, 0};
-    if (PAGED) {
-        const int tk = tid >> 3, gv = v_gv(tid);
-        if (tk < nk_valid) r.bk = bt_row[block_of(p, kbase + tk)];
-        if (4 * gv < nk_valid) r.bv = bt_row[block_of(p, kbase + 4 * gv)];
-    }
+    const int tk = tid >> 3, gv = v_gv(tid);
+    if (tk < nk_valid) r.bk = bt_row[block_of(p, kbase + tk)];
+    if (4 * gv < nk_valid) r.bv = bt_row[block_of(p, kbase + 4 * gv)];
     return r;
 }
 
@@ -270,44 +267,39 @@ __device__ __forceinline__ TileRows fetch_rows(const PrefillParams &p, const int
 // with c = tid & 7.  V share: keys 4g..4g+3 with g = v_gv(tid), dims
 // [4c, 4c+4) with c = v_cv(tid).  Keys at or past nk_valid are not read
 // (zeros; they are masked later).  The dense source goes by DMA instead.
-template <bool PAGED>
 __device__ __forceinline__ void load_tile(const PrefillParams &p, TileRegs &r, TileRows rows,
                                           int h, int kbase, int nk_valid, int tid) {
     const int tk = tid >> 3, ck = tid & 7;
     const int gv = v_gv(tid), cv = v_cv(tid);
-    if (PAGED) {
-        auto in_block = [&](int kpos) { return kpos - block_of(p, kpos) * p.block_size; };
-        const uint8_t *kvh = p.kv + (int64_t)h * p.slot_bytes;
-        r.k[0] = r.k[1] = 0u;
-        r.nk = 0.0f;
-        if (tk < nk_valid) {
-            // Slot rows and row_bytes are below 2^32 and 2^31: one 32 x 32 -> 64-bit multiply.
-            const uint8_t *rp =
-                kvh + (uint64_t)(uint32_t)(rows.bk * p.block_size + in_block(kbase + tk)) *
-                          (uint32_t)p.row_bytes;
-            const uint2 w = *reinterpret_cast<const uint2 *>(rp + 8 * ck);
-            r.k[0] = w.x;
-            r.k[1] = w.y;
-            r.nk = *reinterpret_cast<const float *>(rp + 128);
-        }
-        const uint8_t *vp =
-            kvh + (uint64_t)(uint32_t)(rows.bv * p.block_size + in_block(kbase + 4 * gv)) *
+    auto in_block = [&](int kpos) { return kpos - block_of(p, kpos) * p.block_size; };
+    const uint8_t *kvh = p.kv + (int64_t)h * p.slot_bytes;
+    r.k[0] = r.k[1] = 0u;
+    r.nk = 0.0f;
+    if (tk < nk_valid) {
+        // Slot rows and row_bytes are below 2^32 and 2^31: one 32 x 32 -> 64-bit multiply.
+        const uint8_t *rp =
+            kvh + (uint64_t)(uint32_t)(rows.bk * p.block_size + in_block(kbase + tk)) *
                       (uint32_t)p.row_bytes;
+        const uint2 w = *reinterpret_cast<const uint2 *>(rp + 8 * ck);
+        r.k[0] = w.x;
+        r.k[1] = w.y;
+        r.nk = *reinterpret_cast<const float *>(rp + 128);
+    }
+    const uint8_t *vp =
+        kvh + (uint64_t)(uint32_t)(rows.bv * p.block_size + in_block(kbase + 4 * gv)) *
+                  (uint32_t)p.row_bytes;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            r.v[i] = 0u;
-            r.nv[i] = 0.0f;
-            if (4 * gv + i < nk_valid) {
-                const uint8_t *rp = vp + i * p.row_bytes;
-                r.v[i] = *reinterpret_cast<const uint16_t *>(rp + 64 + 2 * cv);
-                r.nv[i] = *reinterpret_cast<const float *>(rp + 132);
-            }
+    for (int i = 0; i < 4; ++i) {
+        r.v[i] = 0u;
+        r.nv[i] = 0.0f;
+        if (4 * gv + i < nk_valid) {
+            const uint8_t *rp = vp + i * p.row_bytes;
+            r.v[i] = *reinterpret_cast<const uint16_t *>(rp + 64 + 2 * cv);
+            r.nv[i] = *reinterpret_cast<const float *>(rp + 132);
         }
     }
 }
 
-// One code byte's two values fp16(cb[code] * norm) from the per-code table
-// (16 rows x 64 lane columns of fp32).
 // One code byte's two values fp16(cb[code] * norm) from the code-byte table
 // (hi nibble first: the even dim).
 __device__ __forceinline__ uint32_t dq_byte(const uint8_t *lut, uint32_t byte, float norm) {
@@ -666,10 +658,9 @@ prefill_kernel(PrefillParams p) {
         const int k0 = jt0 * kBN, k1 = k0 + kBN;
         issue_dma(jt0);
         if constexpr (PAGED) {
-            load_tile<PAGED>(p, cur, fetch_rows<PAGED>(p, bt_row, k0, min(kBN, kend - k0), tid), h,
-                             k0, min(kBN, kend - k0), tid);
-            if (jt0 + 1 < jt1)
-                rows_next = fetch_rows<PAGED>(p, bt_row, k1, min(kBN, kend - k1), tid);
+            load_tile(p, cur, fetch_rows(p, bt_row, k0, min(kBN, kend - k0), tid), h, k0,
+                      min(kBN, kend - k0), tid);
+            if (jt0 + 1 < jt1) rows_next = fetch_rows(p, bt_row, k1, min(kBN, kend - k1), tid);
         }
     }
     __syncthreads();   // tables visible
@@ -684,9 +675,8 @@ prefill_kernel(PrefillParams p) {
             store_tile(cur, buf, buf + kKTile, lutk, lutv, tid);
             if (j + 1 < jt1) {
                 const int k1 = (j + 1) * kBN, k2 = (j + 2) * kBN;
-                load_tile<PAGED>(p, cur, rows_next, h, k1, min(kBN, kend - k1), tid);
-                if (j + 2 < jt1)
-                    rows_next = fetch_rows<PAGED>(p, bt_row, k2, min(kBN, kend - k2), tid);
+                load_tile(p, cur, rows_next, h, k1, min(kBN, kend - k1), tid);
+                if (j + 2 < jt1) rows_next = fetch_rows(p, bt_row, k2, min(kBN, kend - k2), tid);
             }
         } else {
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
