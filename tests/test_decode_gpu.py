@@ -445,10 +445,10 @@ def test_decode_single_launch_any_heads_and_slots(gpu, codebooks, name, seq_lens
 
 @pytest.mark.parametrize("name,seq_lens,H_kv,gs,levels,slack", [
     ("one_long", [60000] + [1 + 300 * i for i in range(11)], 1, 4, 16, 0),
-    ("empty_between", [0, 8193, 0, 513, 0, 16385, 512, 0, 4096, 1, 1024, 30000], 1, 8, 16, 0),
+    ("empty_between", [0, 8193, 0, 513, 0, 16385, 512, 0, 4096, 1, 1024, 60000], 1, 8, 16, 0),
     ("same_chunk_count", [16384 - 40 * i for i in range(12)], 2, 4, 16, 0),
     ("slack_bound", [900, 33, 2000, 5, 700, 1, 4100, 513], 8, 4, 16, 60000),
-    ("sixty_four", [int(x) for x in np.random.default_rng(12).integers(1, 3000, 63)] + [9000],
+    ("sixty_four", [int(x) for x in np.random.default_rng(12).integers(1, 3000, 63)] + [17000],
      1, 4, 16, 0),
     ("k2v2_two_heads", [int(x) for x in np.random.default_rng(13).integers(1, 9000, 15)] + [20000],
      2, 8, 4, 0),
@@ -463,7 +463,10 @@ def test_decode_slots_by_length(gpu, codebooks, name, seq_lens, H_kv, gs, levels
     launches; twice, bit for bit."""
     from sub0_amd import _native
     print(f"[decode-slots] case={name} B={len(seq_lens)} H_kv={H_kv}", flush=True)
-    assert _native.decode_fused_plan(len(seq_lens), H_kv, slack or max(seq_lens))[1] > 1
+    bound = slack or max(seq_lens)
+    assert _native.decode_fused_plan(len(seq_lens), H_kv, bound)[1] > 1
+    assert (_native.decode_deals_by_length(len(seq_lens), H_kv, bound)
+            is (name not in ("sixty_five", "short")))
     cb = None if levels == 16 else codebooks["lloyd_beta4"].astype(np.float32)
     case = make_decode_case(7600 + len(name), seq_lens, H_kv=H_kv, gs=gs, cb=cb, fill=0xFF)
     got = run_gpu_decode(case, gpu, gs=gs, max_seq_len=slack or None)

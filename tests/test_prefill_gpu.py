@@ -281,24 +281,80 @@ def test_prefill_key_split_padded_query_rows(gpu):
     ([5, 513, 0], [5, 513, 40], 1, 4, 1),
 ])
 def test_prefill_dense_scratch_matches_bridge(gpu, seq_q, seq_k, H_kv, gs, slack):
-    """The dense prefill with its K/V in scratch (rows past a sequence's keys
-    are not written) gives the bits of the two-call bridge, and the checker's
-    output within the tolerance; the scratch starts as NaN."""
+    """The dense prefill with its K/V in scratch gives the bits of the two-call
+    bridge, and the checker's output within the tolerance, through the torch op
+    and the C entry; the C entry's scratch starts as NaN, and the rows past a
+    sequence's keys are neither written nor read."""
+    import ctypes
+    from sub0_amd import _native
+    from sub0_amd.cda._prebuilt_loader import load_torch_ops_library
     print(f"[prefill-dense] seq_q={seq_q} seq_k={seq_k} H_kv={H_kv}", flush=True)
     case = make_prefill_case(6100 + slack, seq_q, seq_k, H_kv=H_kv, gs=gs, fill=0xFF)
     bridge = run_prefill(case, gpu, dense=True)
     q, cache, bt = (_dev(x, gpu) for x in (case.q, case.cache, case.block_table))
     cu, sk, cb = (_dev(x, gpu) for x in (case.cu_q, case.seq_k, case.cb))
-    # What the caching allocator hands the op next: the pattern of a NaN.
-    junk = torch.full((1 << 24,), 0xFF, dtype=torch.uint8, device=gpu)
-    del junk
+    bound, scale = max(seq_k) + slack, float(1 / np.sqrt(128))
     out = torch.full_like(q, float("nan"))
-    torch.ops.cda_hip.prefill_dense(q, cache, bt, cu, sk, cb, cb, out, case.block_size,
-                                    max(seq_q), max(seq_k) + slack, float(1 / np.sqrt(128)))
+    load_torch_ops_library("cda_hip").prefill_dense(q, cache, bt, cu, sk, cb, cb, out,
+                                                     case.block_size, max(seq_q), bound, scale)
+    L = _native.lib()
+    need = L.cda_prefill_dense_workspace_size(len(seq_k), H_kv, bound)
+    scratch = torch.full((need,), 0xFF, dtype=torch.uint8, device=gpu)
+    assert scratch.data_ptr() % 256 == 0
+    out_c = torch.full_like(q, float("nan"))
+    ptr = [ctypes.c_void_p(t.data_ptr()) for t in (q, cache, bt, cu, sk, cb, out_c, scratch)]
+    rc = L.cda_prefill_dense_hadamard(
+        ptr[0], ptr[1], cache.shape[0], cache.shape[2], H_kv, ptr[2], bt.stride(0), ptr[3], ptr[4],
+        len(seq_k), ptr[5], ptr[5], 16, ptr[6], q.shape[0], q.shape[1], case.block_size, max(seq_q),
+        bound, scale, ptr[7], need, ctypes.c_void_p(torch.cuda.current_stream(gpu).cuda_stream))
+    assert rc == 0, L.cda_hip_last_error()
     torch.cuda.synchronize()
-    out = out.cpu().numpy()
-    assert np.array_equal(out.view(np.uint16), bridge.view(np.uint16))
-    check(out, case.expected)
+    for got in (out.cpu().numpy(), out_c.cpu().numpy()):
+        assert np.array_equal(got.view(np.uint16), bridge.view(np.uint16))
+        check(got, case.expected)
+    rows = len(seq_k) * bound * H_kv * 256
+    for half in (scratch[:rows], scratch[need // 2:need // 2 + rows]):
+        half = half.view(len(seq_k), bound, H_kv * 256)
+        for b, n in enumerate(seq_k):
+            assert bool((half[b, n:] == 0xFF).all())
+
+
+@pytest.mark.parametrize("seq_q,seq_k", [([90], [300]), ([16, 3], [5000, 2100]),
+                                         ([300, 40], [300, 513])])
+@pytest.mark.parametrize("path", ["compressed", "dense", "bridge", "hybrid"])
+def test_prefill_block_table_views(gpu, path, seq_q, seq_k):
+    """Column slices of a wider block table, whose other entries name no page and
+    whose last row may end with its storage, give the bits of the contiguous
+    table."""
+    print(f"[prefill-views] path={path} seq_q={seq_q} seq_k={seq_k}", flush=True)
+    from sub0_amd.cda._prebuilt_loader import load_torch_ops_library
+    ops = load_torch_ops_library("cda_hip")
+    case = make_prefill_case(6400, seq_q, seq_k, H_kv=8, gs=4, fill=0xFF)
+    q, cache, bt = (_dev(x, gpu) for x in (case.q, case.cache, case.block_table))
+    cu, sk, cb = (_dev(x, gpu) for x in (case.cu_q, case.seq_k, case.cb))
+    bs, mq, mk, scale = case.block_size, max(seq_q), max(seq_k), float(1 / np.sqrt(128))
+    k, v = (_dev(synth.normal_f16(6410 + i, (q.shape[0], 8, 128)), gpu) for i in range(2))
+
+    def run(table):
+        out = torch.full_like(q, float("nan"))
+        if path == "compressed":
+            ops.prefill(q, cache, table, cu, sk, cb, cb, out, bs, mq, scale, mk)
+        elif path == "dense":
+            ops.prefill_dense(q, cache, table, cu, sk, cb, cb, out, bs, mq, mk, scale)
+        elif path == "hybrid":
+            ops.prefill_hybrid(q, k, v, cache, table, cu, sk, cb, cb, out, bs, mq, mk, scale)
+        else:
+            return torch.stack(ops.paged_to_dense(cache, table, sk, cb, cb, bs, mk))
+        return out
+    want = run(bt)
+    B, W = bt.shape
+    for first in (0, 21):
+        wide = torch.full((B, W + 21), 0x7FFFFFFF, dtype=torch.int32, device=gpu)
+        view = wide[:, first:first + W]
+        view.copy_(bt)
+        assert torch.equal(run(view).view(torch.int16), want.view(torch.int16))
+    if path in ("compressed", "dense"):
+        check(want.cpu().numpy(), case.expected)
 
 
 @pytest.mark.parametrize("seq_k", [[1], [70, 64], [127], [129, 65, 200]])
