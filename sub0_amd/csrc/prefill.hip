@@ -1443,9 +1443,8 @@ extern "C" int cda_prefill_dense_hadamard(const void *q, const void *kv_cache, i
     (void)num_slots;
     CDA_REQUIRE(levels_v == 16 || levels_v == 4,
                 "cda_prefill_dense_hadamard: K4V4 or K4V2 caches (V codebook of 16 or 4 levels)");
-    CDA_REQUIRE(max_seq_len > 0 || B == 0 || max_query_len == 0,
-                "cda_prefill_dense_hadamard: max_seq_len must be > 0");
-    if (B == 0 || max_query_len == 0) return CDA_OK;
+    CDA_REQUIRE(max_seq_len > 0 || B == 0, "cda_prefill_dense_hadamard: max_seq_len must be > 0");
+    if (B == 0) return CDA_OK;
     const size_t need = cda_prefill_dense_workspace_size(B, H_kv, max_seq_len);
     if (!workspace || workspace_bytes < need || need == 0 || ((uintptr_t)workspace & 255))
         return fail(CDA_E_WORKSPACE, "cda_prefill_dense_hadamard: workspace missing, misaligned "

@@ -214,6 +214,20 @@ def test_prefill_arguments_are_rejected_before_launch():
     assert call(144, 16, P(260)) == -1 and b"aligned" in L.cda_hip_last_error()
 
 
+def test_prefill_dense_checks_without_queries():
+    """max_query_len 0 does not skip the checks of the loader and the attention
+    that the two-call bridge made (a slot too small for the layout)."""
+    from sub0_amd import _native
+    L = _native.lib()
+    d = ctypes.c_void_p(256)
+
+    def call(slot_bytes, max_query_len):
+        return L.cda_prefill_dense_hadamard(d, d, 64, slot_bytes, 8, d, 4, d, d, 1, d, d, 16, d, 8,
+                                            32, 16, max_query_len, 64, 0.1, d, 1 << 30, None)
+    for max_query_len in (8, 0):
+        assert call(128, max_query_len) == -1 and b"slot" in L.cda_hip_last_error()
+
+
 def test_python_binding_refuses_cpu_tensors():
     import torch
     from sub0_amd import _native
