@@ -700,6 +700,7 @@ decode_stream_kernel(SplitParams p) {
     if (lane < L) cb_lane = SQK ? p.cb_v[lane] : p.cb_k[lane];
     if (TWO && lane >= 16 && lane < 16 + L) cb_lane = p.cb_v[lane - 16];
     int seq_len;
+    bool dealt = false;
     if constexpr (SLOTS) {
         // Sequences of one length keep the even split, for which the loads
         // above went out.  Otherwise a split is k chunks of 512 tokens (64 per
@@ -726,6 +727,7 @@ decode_stream_kernel(SplitParams p) {
             if (512 * k < tile_n) {
                 tile_n = 512 * k;
                 wave_tokens = 64 * k;
+                dealt = true;
                 const int n_l = max(1, (t_l + k - 1) / k);
                 int first = 0;
                 for (b = 0; b < p.B; ++b) {
@@ -778,10 +780,11 @@ decode_stream_kernel(SplitParams p) {
         // above the lengths (a captured graph's) would leave them all to the
         // first wave or two, 6 x 17418 tokens under a bound of 128K, 8 KV heads,
         // 149 -> 109 us, 24 x 2654 with 512-byte slots 277 -> 86.  Not for one
-        // chunk less, which the second read of the table row costs; marked unlikely,
-        // or one chunk per wave takes 0.3 us more (8 queries per head, 895 tokens 16.4).
+        // chunk less, which the second read of the table row costs, nor where the
+        // slots were dealt by length; marked unlikely, or one chunk per wave takes
+        // 0.3 us more (8 queries per head, 895 tokens 16.4).
         const int share = ((end - start + 64 * kWaves - 1) / (64 * kWaves)) * 64;
-        if (__builtin_expect(wave_tokens > 128 && share + 128 <= wave_tokens, 0)) {
+        if (__builtin_expect(!dealt && wave_tokens > 128 && share + 128 <= wave_tokens, 0)) {
             wave_tokens = share;
             load_pages();
         }
