@@ -593,7 +593,10 @@ __device__ __forceinline__ uint32_t bfi(uint32_t m, uint32_t a, uint32_t b) {
 // the V entry in the second, so a table read is the same instruction with an
 // offset of 128.  With half the columns two lanes of a read share each bank:
 // 4.0 instead of 2.9 cycles per ds_read_b64 and CU, 8.2 instead of 4.1 per
-// ds_read_b128 (2-bit codes), which is why one codebook keeps the full row.
+// ds_read_b128 (2-bit codes), which is why one codebook keeps the full row: 32 x
+// 64K tokens 524 us with one, 540 with two, equal bits or not (2-bit codes 453 /
+// 474), 1 x 4K 14.6 / 14.7.  The three launches took 544 with two equal ones, which
+// they compare on the device, and 618 with different ones (491 / 727; 22.1 / 23.3).
 template <int GS, int L, bool SQK = false, bool FUSED = false, bool TWO = false,
           bool SLOTS = false>
 __global__ void __launch_bounds__(kThreads, 1)
