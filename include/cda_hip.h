@@ -258,7 +258,7 @@ int cda_prefill_paged_hadamard(const void *q, const void *kv_cache, int64_t num_
 
 /* Same operation as cda_prefill_paged_hadamard, for short query chunks over
  * long contexts: when the query blocks x sequences x KV heads leave most CUs
- * idle (fewer than 256 workgroups), the keys of each query block are split
+ * idle (fewer workgroups than CUs), the keys of each query block are split
  * (at least 256 keys per split, at most 64 splits); the splits write
  * unnormalised partials (O, m, l) into the workspace and a combine kernel
  * merges them (attention.py:239-272) before the fp16 rounding of O_rot and
@@ -268,7 +268,8 @@ int cda_prefill_paged_hadamard(const void *q, const void *kv_cache, int64_t num_
  *   max_seq_len:   upper bound of seq_lens[b] (the longest key range).
  *   workspace:     device scratch, 256-byte aligned, of at least
  *                  cda_prefill_workspace_size(B, T, H_q, H_kv, max_query_len,
- *                  max_seq_len) bytes (0: no split, workspace may be NULL).
+ *                  max_seq_len) bytes (0: no split, workspace may be NULL); one
+ *                  sized for more rows T is enough for fewer.
  * Calls sharing one workspace must not overlap.
  */
 size_t cda_prefill_workspace_size(int B, int T, int H_q, int H_kv, int max_query_len,

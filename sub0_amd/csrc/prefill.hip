@@ -1047,13 +1047,22 @@ int launch_prefill(const PrefillParams &p, int B, int max_q, hipStream_t st, con
 // grid a little over a round nearly fits it: 12 x 64 over 10K-16K, 3 splits of 86
 // tiles 257 us; 7 x 64, 5 of 52 155 (4 of 65: 167).  With equal counts, which a
 // plan that cannot see them has to expect, the same grids take two full rounds:
-// 16K each, 425 (five: 290) and 262 (four: 175).  Nor can it see query counts:
-// 3 x 194-389 queries over 2.5K-4K, hybrid, 144 workgroups of which 128 have
-// queries, take 3 splits (153 us) where 2 fit one round (135).
+// 16K each, 425 (five: 290) and 262 (four: 175).
+//
+// B * max_q bounds the query blocks; the T query rows tell how many there are
+// where the counts differ: the longest sequence's, and of the others' rows T -
+// max_q one more half block each on average (T = B * max_q leaves no doubt).  If the
+// count that fills the CUs by the bound then fits one round, it is taken: 3 x
+// 194-389 queries over 2.5K-4K, hybrid, 144 workgroups by the bound and 120 with
+// queries, 2 splits 128 us, the 3 that the bound asks for 153.  Only where every
+// XCD has whole heads: with fewer the longest sequence's XCDs are over a round (4
+// x 77-155 queries over 3.3K, 4 KV heads: 89 us against 64).  Without `by_rows`
+// the plan depends on the bound alone: a workspace sized for more rows need not
+// hold the other's partials.
 constexpr int kMaxKsplit = 64;
 static_assert(kMaxKsplit <= 64, "prefill_combine_kernel: one lane per split");
-void prefill_ksplit_plan(int B, int H_q, int H_kv, int max_q, int max_k, int *n_split,
-                         int *split_tiles, bool always_merged = false) {
+void prefill_ksplit_plan(int B, int T, int H_q, int H_kv, int max_q, int max_k, int *n_split,
+                         int *split_tiles, bool by_rows, bool always_merged = false) {
     // always_merged: the hybrid, whose two parts are merged from partials also
     // where neither is split, and have half of the merge's splits each.
     const int max_split = always_merged ? kMaxKsplit / 2 : kMaxKsplit;
@@ -1064,6 +1073,21 @@ void prefill_ksplit_plan(int B, int H_q, int H_kv, int max_q, int max_k, int *n_
     *split_tiles = tiles;
     const int64_t cus = num_cus();
     if (wgs <= 0 || wgs >= cus) return;
+    const int fill = (int)std::min<int64_t>((cus + wgs - 1) / wgs, std::min(tiles / 4, max_split));
+    if (by_rows && H_kv % (int)kXcds == 0 && fill > 1 && wgs * fill > cus &&
+        T < (int64_t)B * max_q) {
+        // Expected query blocks, in 1 / (2 * qb) of one.
+        const int64_t rest = std::max<int64_t>(T - max_q, 0), others = B - 1;
+        const int64_t nb = (max_q + qb - 1) / qb, lo = (rest + qb - 1) / qb;
+        const int64_t hi = std::min(nb * others, std::max<int64_t>(rest - others, 0) / qb +
+                                                     std::min(others, rest));
+        const int64_t mean = std::min(std::max(2 * rest + others * qb, 2 * qb * lo), 2 * qb * hi);
+        if ((2 * qb * nb + mean) * H_kv * fill <= 2 * qb * cus) {
+            *split_tiles = (tiles + fill - 1) / fill;
+            *n_split = (tiles + *split_tiles - 1) / *split_tiles;
+            return;
+        }
+    }
     constexpr int kFixed = 3;                              // set-up and epilogue, in tiles
     constexpr int kRowsPerTile = 15000;                    // partial rows moved in a tile's time
     const int64_t rows = (int64_t)B * max_q * H_q;
@@ -1139,7 +1163,9 @@ int prefill_paged_impl(const char *fn, const void *q, const void *kv_cache, int 
     CDA_REQUIRE(T > 0 || max_query_len == 0, std::string(fn) + ": T must be the number of query rows");
     if (max_seq_len >= 0) {
         int ns, per;
-        prefill_ksplit_plan(B, H_q, H_kv, max_query_len, max_seq_len, &ns, &per);
+        prefill_ksplit_plan(B, T, H_q, H_kv, max_query_len, max_seq_len, &ns, &per, true);
+        if (ns > 1 && workspace_bytes < prefill_ws_bytes(T, H_q, ns))
+            prefill_ksplit_plan(B, T, H_q, H_kv, max_query_len, max_seq_len, &ns, &per, false);
         if (ns > 1) {
             CDA_REQUIRE(T > 0, std::string(fn) + ": T must be the number of query rows");
             const size_t need = prefill_ws_bytes(T, H_q, ns);
@@ -1178,7 +1204,7 @@ extern "C" size_t cda_prefill_workspace_size(int B, int T, int H_q, int H_kv, in
         (H_q / H_kv != 4 && H_q / H_kv != 8) || max_query_len <= 0 || max_seq_len <= 0)
         return 0;
     int ns, per;
-    prefill_ksplit_plan(B, H_q, H_kv, max_query_len, max_seq_len, &ns, &per);
+    prefill_ksplit_plan(B, T, H_q, H_kv, max_query_len, max_seq_len, &ns, &per, true);
     return ns > 1 ? prefill_ws_bytes(T, H_q, ns) : 0;
 }
 
@@ -1492,11 +1518,12 @@ struct HybridPlan {
     size_t part_bytes, kv_bytes;
 };
 
-HybridPlan hybrid_plan(int B, int T, int H_q, int H_kv, int max_query_len, int max_seq_len) {
+HybridPlan hybrid_plan(int B, int T, int H_q, int H_kv, int max_query_len, int max_seq_len,
+                       bool by_rows) {
     HybridPlan h{};
-    prefill_ksplit_plan(B, H_q, H_kv, max_query_len, std::max(1, max_seq_len - 1), &h.na,
-                        &h.na_tiles, true);
-    prefill_ksplit_plan(B, H_q, H_kv, max_query_len, max_query_len, &h.nb, &h.nb_tiles,
+    prefill_ksplit_plan(B, T, H_q, H_kv, max_query_len, std::max(1, max_seq_len - 1), &h.na,
+                        &h.na_tiles, by_rows, true);
+    prefill_ksplit_plan(B, T, H_q, H_kv, max_query_len, max_query_len, &h.nb, &h.nb_tiles, by_rows,
                         true);
     h.part_bytes = prefill_ws_bytes(T, H_q, h.na + h.nb);
     h.kv_bytes = (((size_t)T * H_kv * kD * 2) + 255) & ~(size_t)255;
@@ -1510,7 +1537,7 @@ extern "C" size_t cda_prefill_hybrid_workspace_size(int B, int T, int H_q, int H
     if (B <= 0 || T <= 0 || H_q <= 0 || H_kv <= 0 || H_q % H_kv != 0 ||
         (H_q / H_kv != 4 && H_q / H_kv != 8) || max_query_len <= 0 || max_seq_len <= 0)
         return 0;
-    const HybridPlan h = hybrid_plan(B, T, H_q, H_kv, max_query_len, max_seq_len);
+    const HybridPlan h = hybrid_plan(B, T, H_q, H_kv, max_query_len, max_seq_len, true);
     return h.part_bytes + 2 * h.kv_bytes;
 }
 
@@ -1542,7 +1569,9 @@ extern "C" int cda_prefill_hybrid_rawkv(const void *q, const void *k_new, const 
                 "8-byte aligned");
     if (B == 0 || max_query_len == 0) return CDA_OK;
     CDA_REQUIRE(T > 0, "cda_prefill_hybrid_rawkv: T must be the number of query rows");
-    const HybridPlan h = hybrid_plan(B, T, H_q, H_kv, max_query_len, std::max(1, max_seq_len));
+    HybridPlan h = hybrid_plan(B, T, H_q, H_kv, max_query_len, std::max(1, max_seq_len), true);
+    if (workspace_bytes < h.part_bytes + 2 * h.kv_bytes)
+        h = hybrid_plan(B, T, H_q, H_kv, max_query_len, std::max(1, max_seq_len), false);
     const size_t need = h.part_bytes + 2 * h.kv_bytes;
     if (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 255))
         return fail(CDA_E_WORKSPACE, "cda_prefill_hybrid_rawkv: workspace missing, misaligned or "

@@ -168,6 +168,11 @@ def test_prefill_key_split_plan():
     # workgroups -> unsplit, not 8 splits.
     assert ws(12, 768, 32, 8, 64, 16448) == 5 * 768 * 32 * 128 * 4 + 5 * 768 * 32 * 2 * 4
     assert ws(28, 1792, 32, 8, 64, 16448) == 0
+    # Fewer rows than the bound: 389, 245, 215 queries over 4.4K keys, 144
+    # workgroups by the bound but about 15 blocks x 8 heads: 2 splits fit one round,
+    # where equal counts (21 blocks) take 3 of 23 tiles in two.
+    assert ws(3, 849, 32, 8, 389, 4400) == 2 * 849 * 32 * 128 * 4 + 2 * 849 * 32 * 2 * 4
+    assert ws(3, 1167, 32, 8, 389, 4400) == 3 * 1167 * 32 * 128 * 4 + 3 * 1167 * 32 * 2 * 4
     assert ws(8, 8 * 4096, 32, 8, 4096, 8192) == 0   # config-3-sized grid fills the chip
     assert ws(0, 0, 32, 8, 16, 16384) == 0
     assert ws(1, 16, 32, 5, 16, 16384) == 0          # group size not 4 or 8

@@ -275,6 +275,50 @@ def test_prefill_key_split_padded_query_rows(gpu):
     assert np.isnan(out[12:]).all()
 
 
+@pytest.mark.parametrize("hybrid", [False, True], ids=["paged", "hybrid"])
+def test_prefill_key_split_by_rows(gpu, hybrid):
+    """Query counts below the bound: the rows tell that two splits fit one round
+    (331, 200 and 180 queries; equal counts stay unsplit).  A workspace sized for
+    equal counts is still enough: the call then takes the bound's plan."""
+    import ctypes
+    from sub0_amd import _native
+    from tests.cases import make_hybrid_case
+    print(f"[prefill-split] by rows hybrid={hybrid}", flush=True)
+    seq_q, seq_k = [331, 200, 180], [512, 500, 400]
+    if hybrid:
+        seq_k = [q + k for q, k in zip(seq_q, seq_k)]
+    make = make_hybrid_case if hybrid else make_prefill_case
+    case = make(6500, seq_q, seq_k, H_kv=8, gs=4)
+    T, L = sum(seq_q), _native.lib()
+    size = L.cda_prefill_hybrid_workspace_size if hybrid else L.cda_prefill_workspace_size
+    need, equal = (size(3, t, 32, 8, max(seq_q), max(seq_k)) for t in (T, 3 * max(seq_q)))
+    if not hybrid:
+        assert need > 0 and equal == 0
+    q, cache, bt = (_dev(x, gpu) for x in (case.q, case.cache, case.block_table))
+    cu, sk, cb = (_dev(x, gpu) for x in (case.cu_q, case.seq_k, case.cb))
+    kn, vn = (_dev(case.k_new, gpu), _dev(case.v_new, gpu)) if hybrid else (None, None)
+    P = [ctypes.c_void_p(t.data_ptr()) for t in (q, cache, bt, cu, sk, cb)]
+    stream = ctypes.c_void_p(torch.cuda.current_stream(gpu).cuda_stream)
+    scale = float(1 / np.sqrt(128))
+    for nbytes in (need, equal):
+        ws = torch.full((max(nbytes, 1),), 0xFF, dtype=torch.uint8, device=gpu)
+        w = ctypes.c_void_p(ws.data_ptr() if nbytes else None)
+        out = torch.full_like(q, float("nan"))
+        o = ctypes.c_void_p(out.data_ptr())
+        tail = (o, T, 32, case.block_size, max(seq_q), max(seq_k), scale, w, nbytes, stream)
+        if hybrid:
+            rc = L.cda_prefill_hybrid_rawkv(
+                P[0], ctypes.c_void_p(kn.data_ptr()), ctypes.c_void_p(vn.data_ptr()), P[1],
+                cache.shape[0], cache.shape[2], 8, P[2], bt.stride(0), P[3], P[4], 3, P[5], P[5], 16,
+                *tail)
+        else:
+            rc = L.cda_prefill_paged_hadamard_ws(P[0], P[1], cache.shape[0], cache.shape[2], 8, P[2],
+                                                 bt.stride(0), P[3], P[4], 3, P[5], P[5], 16, *tail)
+        assert rc == 0, L.cda_hip_last_error()
+        torch.cuda.synchronize()
+        check(out.cpu().numpy(), case.expected)
+
+
 @pytest.mark.parametrize("seq_q,seq_k,H_kv,gs,slack", [
     ([300, 1, 77], [300, 1000, 77], 8, 4, 0),
     ([64], [65], 2, 8, 63),
