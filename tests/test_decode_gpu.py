@@ -583,7 +583,7 @@ def test_decode_pages_past_2_31_rows(gpu, codebooks):
 ])
 def test_decode_under_a_loose_bound(gpu, codebooks, name, seq_lens, H_kv, gs, levels, slot):
     """Lengths far below max_seq_len (131072), where the waves of a workgroup
-    share what there is instead of their part of the bound: the checker's output,
+    share what there is instead of their part of the bound: the oracle's output,
     and the tight bound's."""
     print(f"[decode-loose] case={name} B={len(seq_lens)} H_kv={H_kv}", flush=True)
     cb = None if levels == 16 else codebooks["lloyd_beta4"].astype(np.float32)

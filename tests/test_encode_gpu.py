@@ -197,7 +197,7 @@ def test_encode_mfma_form_edges(gpu, codebooks, levels, T, H_kv):
 @pytest.mark.parametrize("levels,T,H_kv", [(16, 40, 8), (16, 700, 8), (4, 1367, 3)])
 def test_encode_non_finite_vectors(gpu, codebooks, levels, T, H_kv):
     """Vectors with infinities and NaNs among finite ones, in the 16-lane form
-    (40 tokens) and the MFMA form: the checker's codes for all of them, its norm
+    (40 tokens) and the MFMA form: the oracle's codes for all of them, its norm
     bits for the finite ones, also beside a non-finite one in the same wave, and
     its infinite or NaN norm for the others."""
     print(f"[encode] non-finite levels={levels} T={T} H_kv={H_kv}", flush=True)

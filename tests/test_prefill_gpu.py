@@ -326,7 +326,7 @@ def test_prefill_key_split_by_rows(gpu, hybrid):
 ])
 def test_prefill_dense_scratch_matches_bridge(gpu, seq_q, seq_k, H_kv, gs, slack):
     """The dense prefill with its K/V in scratch gives the bits of the two-call
-    bridge, and the checker's output within the tolerance, through the torch op
+    bridge, and the oracle's output within the tolerance, through the torch op
     and the C entry; the C entry's scratch starts as NaN, and the rows past a
     sequence's keys are neither written nor read."""
     import ctypes
